@@ -16,15 +16,23 @@
 // of several tiles per wavefront) first resolve all of them into an LDS column table partitioned by tier, so every
 // tile holds rows of one tier and padding columns cost nothing; a block of one tile per wavefront resolves its own
 // tile.  A tile's K and V rows are dequantized into the wavefront's LDS rows as bf16, then QK^T and P.V run as bf16
-// 16x16x16 matrix-core steps with fp32 accumulation:
-//   S^T[row][head] = K[row][:] . Q[head][:]   (A = K tile, B = Q^T; 16 steps over the 256 channels)
-//   O[head][ch]   += P[head][row] V[row][ch]  (A = P straight from S^T's accumulator layout as bf16 high part
-//                                               + bf16 remainder, B = V tile by the transposing LDS read)
+// 16x16x32 matrix-core steps with fp32 accumulation:
+//   S^T[row][head] = K[row][:] . Q[head][:]   (A = K tile, B = Q^T in registers; 8 steps over the 256 channels)
+//   O[head][ch]   += P[head][row] V[row][ch]  (A = P straight from S^T's accumulator layout: bf16 high parts in one
+//                                               half of the 32 k indices, bf16 remainders in the other; B = the 16 V
+//                                               rows in both halves, by the transposing LDS read)
 // with an online softmax across a wavefront's tiles.  The 16 accumulator rows hold up to 16 q heads per KV head
 // (GQA 8 of the configurations, 12 of the served model).  The 4 wavefronts merge through LDS, 8 heads per pass.
 // In decode, columns c of request b attend when c < the request's valid count (cu_k[b + 1] - cu_k[b]) and
 // 0 <= indices[b][c] < seq_lens[b] - the columns the reference's gather writes and its attention reads when the
 // valid positions come first (the indexer pads with -1 at the end).
+//
+// What bounds it: instruction issue, most of it the exact dequantization (per tile ~460 vector instructions, 24
+// products, 72 LDS accesses, 32 loads).  Two rows per wavefront instruction (8 channels a lane), no products with
+// smoothing factors of 1, 32-deep products (the matrix pipe takes as long for a 16-deep one) and the next tile's loads
+// in flight beside a tile's work took the paged prefix chunk (60,000 + 1,024 positions, top 2,051, 12 heads) from 237 to
+// 169 us, the dense slot decode (4 x 65,536) from 70 to 55 us and the top-k decode (8 x 2,051, 12 layers) from 234 to
+// 200 us, against one row per instruction, 16-deep products and loads waited for at the head of each tile.
 //
 // Kinds (the compact gather's codes): 0 INT8-G pool, 1 INT4-G32 pool, 2 tiered (INT8-G ring over INT4-G32 rows,
 // owner test).
@@ -42,8 +50,9 @@ constexpr int kCols = kWaves * kRows;  // selected columns per block (one partia
 constexpr int kHeads = 16;         // q heads per KV head the tile holds (rows beyond the group are zero)
 constexpr int kKPitch = kD + 8;    // bf16 per K row in LDS (the pad spreads a column of rows over the banks)
 
-typedef short bf4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) bf4 lds_v4s;
+typedef short s4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s4v lds_v4s;
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 struct SparseArgs {
@@ -112,7 +121,7 @@ KVT_DEV int64_t idx_value(const IdxWords& x) {
   return (int64_t)(((uint64_t)top << 32) | x.lo);
 }
 
-KVT_DEV f4 mfma_bf16(bf4 a, bf4 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+KVT_DEV f4 mfma_bf16(bf8 a, bf8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // bf16 pair (round to nearest even, one v_cvt_pk_bf16_f32): lo in bits 0-15.
 KVT_DEV uint32_t bf16x2(float lo, float hi) {
@@ -125,14 +134,15 @@ KVT_DEV __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
-// Channels 4 lane .. 4 lane + 3 of one row, dequantized: bf16((c * s) * sm) for code c, the row's fp16 scale s
-// (bits sbits) and the channel's smoothing factor sm, as the gathers write them.  INT8 rows give 4 codes in the
-// loaded word; INT4 rows the 16-bit half (lane & 1) of the word holding channel pairs 4 (lane >> 1) .. + 3 (low
-// nibble = even channel), stored as c + 8.  A code with offset o (c + o >= 0) goes into the mantissa of an fp16 magic
-// value h = 1024 + (c + o) (v_perm_b32 for bytes, v_and_or_b32 for nibble pairs); v_fma_mix_f32 converts h and s and
-// computes h * s - (1024 + o) * s in one rounding, whose exact value c * s is representable (4 or 8 bits times the
-// scale's 11), so the fp32 product equals the plain c * s; the smoothing factor then multiplies in fp32 and
-// v_cvt_pk_bf16_f32 rounds each pair to nearest even.
+// Eight channels of one row, dequantized: bf16((c * s) * sm) for code c, the row's fp16 scale s (bits sbits) and the
+// channel's smoothing factor sm, as the gathers write them.  INT8 rows give 8 bytes of codes, INT4 rows 4 (byte j =
+// channel 2 j in the low nibble, 2 j + 1 in the high one, stored as c + 8).  A code with offset o (c + o >= 0) goes
+// into the mantissa of an fp16 magic value h = 1024 + (c + o) (v_perm_b32 for bytes, v_and_or_b32 for nibbles), in
+// pairs of channels (0, 2), (1, 3), (4, 6), (5, 7); v_fma_mix_f32 converts h and s and computes
+// h * s - (1024 + o) * s in one rounding, whose exact value c * s is representable (4 or 8 bits times the scale's
+// 11), so the fp32 product equals the plain c * s; the smoothing factor then multiplies in fp32 (SM; a product with 1
+// changes nothing, so identity factors take the body without it) and v_cvt_pk_bf16_f32 rounds each pair to nearest
+// even.
 KVT_DEV uint32_t and_or(uint32_t x, uint32_t m, uint32_t o) {
   uint32_t r;
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(m), "v"(o));
@@ -142,159 +152,168 @@ KVT_DEV float mix(uint32_t w, int half, _Float16 s, float c) {
   typedef _Float16 h2v __attribute__((ext_vector_type(2)));
   return fmaf((float)__builtin_bit_cast(h2v, w)[half], (float)s, c);
 }
-KVT_DEV uint2 dequant4(bool hot, uint32_t w, uint32_t sbits, int lane, const float sm[4]) {
+KVT_DEV void magic8(uint2 w, uint32_t m[4]) {
+  const uint32_t u = w.x ^ 0x80808080u, v = w.y ^ 0x80808080u;
+  m[0] = __builtin_amdgcn_perm(0x64646464u, u, 0x04020400u);
+  m[1] = __builtin_amdgcn_perm(0x64646464u, u, 0x04030401u);
+  m[2] = __builtin_amdgcn_perm(0x64646464u, v, 0x04020400u);
+  m[3] = __builtin_amdgcn_perm(0x64646464u, v, 0x04030401u);
+}
+KVT_DEV void magic4(uint32_t w, uint32_t m[4]) {   // pairs (0, 4), (1, 5), (2, 6), (3, 7): one instruction less
+  m[0] = and_or(w, 0x000F000Fu, 0x64006400u);
+  m[1] = and_or(w >> 4, 0x000F000Fu, 0x64006400u);
+  m[2] = and_or(w >> 8, 0x000F000Fu, 0x64006400u);
+  m[3] = and_or(w >> 12, 0x000F000Fu, 0x64006400u);
+}
+KVT_DEV void magic4_as8(uint32_t w, uint32_t m[4]) {   // in magic8's pairs
+  const uint32_t a = __builtin_amdgcn_perm(0u, w, 0x0c010c00u);   // bytes 0, 1 in the low byte of each half
+  const uint32_t b = __builtin_amdgcn_perm(0u, w, 0x0c030c02u);
+  m[0] = and_or(a, 0x000F000Fu, 0x64006400u);
+  m[1] = and_or(a >> 4, 0x000F000Fu, 0x64006400u);
+  m[2] = and_or(b, 0x000F000Fu, 0x64006400u);
+  m[3] = and_or(b >> 4, 0x000F000Fu, 0x64006400u);
+}
+// offset: 1024 + o (exact products, as the scale's 11 bits times 1032 or 1152 = 9 * 128 fit fp32)
+template <bool SM, bool PAIRS4>
+KVT_DEV uint4 rows_bf16(const uint32_t m[4], uint32_t sbits, float offset, const uint4& sm) {
   const _Float16 s = __builtin_bit_cast(_Float16, (uint16_t)(sbits & 0xffffu));
-  uint32_t a, b;   // fp16 magic pairs: hot a = channels (0, 2), b = (1, 3); INT4 a = (0, 1), b = (2, 3)
-  float c;
-  if (hot) {
-    const uint32_t u = w ^ 0x80808080u;
-    a = __builtin_amdgcn_perm(0x64646464u, u, 0x04020400u);
-    b = __builtin_amdgcn_perm(0x64646464u, u, 0x04030401u);
-    c = -1152.0f * (float)s;
-  } else {
-    const uint32_t h = (w >> (16 * (lane & 1))) & 0xffffu;
-    const uint32_t x = h | (h << 12);   // nibble 1 at bits 16-19, nibble 3 at bits 24-27
-    a = and_or(x, 0x000F000Fu, 0x64006400u);
-    b = and_or(x >> 8, 0x000F000Fu, 0x64006400u);
-    c = -1032.0f * (float)s;
+  const float c = fmaf((float)s, -offset, 0.0f);   // (one v_fma_mix_f32)
+  float x[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int lo = PAIRS4 ? j : 4 * (j >> 1) + (j & 1);
+    x[lo] = mix(m[j], 0, s, c), x[lo + (PAIRS4 ? 4 : 2)] = mix(m[j], 1, s, c);
   }
-  float v[4];
-  if (hot) {
-    v[0] = mix(a, 0, s, c), v[1] = mix(b, 0, s, c), v[2] = mix(a, 1, s, c), v[3] = mix(b, 1, s, c);
-  } else {
-    v[0] = mix(a, 0, s, c), v[1] = mix(a, 1, s, c), v[2] = mix(b, 0, s, c), v[3] = mix(b, 1, s, c);
+  if constexpr (SM) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t w = i < 2 ? sm.x : i < 4 ? sm.y : i < 6 ? sm.z : sm.w;
+      x[i] *= f16_bits_to_f32((uint16_t)(w >> (16 * (i & 1))));
+    }
   }
-  return uint2{bf16x2(v[0] * sm[0], v[1] * sm[1]), bf16x2(v[2] * sm[2], v[3] * sm[3])};
+  return uint4{bf16x2(x[0], x[1]), bf16x2(x[2], x[3]), bf16x2(x[4], x[5]), bf16x2(x[6], x[7])};
 }
 
-// One tile's raw row data for this lane (channels 4 lane .. + 3 of K and V, and their scales).
-struct TileLoads {
-  uint32_t kw[kRows], vw[kRows], ks[kRows], vs[kRows];
-  int fl[kRows];
+// The raw data of a tile: a wavefront takes two rows at once, lanes 0-31 row 2 i and lanes 32-63 row 2 i + 1, each
+// lane 8 channels (8 (lane & 31) ..) -- half the loads and LDS stores of one row per wavefront, and no shuffling of
+// half-used words.
+constexpr int kPairs = kRows / 2;
+struct Raw {
+  uint2 w8[kPairs];      // INT8 codes
+  uint32_t w4[kPairs];   // INT4 codes
+  uint32_t s8[kPairs], s4[kPairs];
 };
 
-constexpr uint32_t kNoRow = 0x80000000u;   // a row offset past every buffer: its loads return zero
+// A row of the pools as one word: row * H + head (below 2^24), bit 30 set for a ring (INT8) row of a mixed tile.
+// kNoRow (not attended): every byte offset formed from it lies past the buffers (all below 2^31 bytes) without
+// wrapping, so its loads return zeros.
+constexpr uint32_t kNoRow = 0xffffffffu;
+constexpr uint32_t kHotBit = 1u << 30;
 
 // Buffer resources over whole tensors (byte offsets are 32-bit: the launcher checks the sizes).
 struct PoolRsrc {
   __amdgpu_buffer_rsrc_t k8, v8, ks8, vs8, k4, v4, ks4, vs4;
 };
 
-// Issue the loads of the wavefront's tile: row r's byte offsets (codes and scales, in the row's tier) come from
-// lane r by readlane and go in the scalar offset of the loads, so every row costs a few scalar instructions and no
-// vector address math; the lane offsets are fixed per tier.
-// TIERS: the tile's rows are all INT8 (kRowsInt8), all INT4 (kRowsInt4) or each in its own tier (kRowsMixed: a
-// wavefront-uniform branch per row).
+// TIERS: the tile's rows are all INT8 (kRowsInt8), all INT4 (kRowsInt4) or each in its own tier (kRowsMixed: both
+// tiers' loads are issued, the row's absent tier at an offset past its buffer, and the magic words selected).
 enum { kRowsInt8 = 0, kRowsInt4 = 1, kRowsMixed = 2 };
 
+// Issue the loads of K or V of a tile whose row words (of this lane's half: rows 2 i + (lane >> 5)) are e[i].
 template <int G8, int TIERS>
-KVT_DEV void issue_tile(const PoolRsrc& P, int flags, uint32_t coff, uint32_t soff, int lane, TileLoads& L) {
-  const uint32_t off8 = 4u * lane, off4 = 4u * (lane >> 1);
-  const uint32_t soff8 = 2u * ((4u * lane) / G8), soff4 = 2u * (lane >> 3);
+KVT_DEV void issue_rows(__amdgpu_buffer_rsrc_t r8, __amdgpu_buffer_rsrc_t rs8, __amdgpu_buffer_rsrc_t r4,
+                        __amdgpu_buffer_rsrc_t rs4, const uint32_t e[kPairs], int lane, Raw& R) {
+  constexpr uint32_t kSh8 = kD / G8 * 2;   // scale bytes of an INT8 row
+  const uint32_t g = (uint32_t)lane & 31u;
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int f = TIERS == kRowsMixed ? __builtin_amdgcn_readlane(flags, r) : (TIERS == kRowsInt8 ? 2 : 0);
-    L.fl[r] = f;
-    const uint32_t co = (uint32_t)__builtin_amdgcn_readlane((int)coff, r);
-    const uint32_t so = (uint32_t)__builtin_amdgcn_readlane((int)soff, r);
-    if ((f & 2) != 0) {
-      L.kw[r] = __builtin_amdgcn_raw_buffer_load_b32(P.k8, off8, co, 0);
-      L.vw[r] = __builtin_amdgcn_raw_buffer_load_b32(P.v8, off8, co, 0);
-      L.ks[r] = __builtin_amdgcn_raw_buffer_load_b16(P.ks8, soff8, so, 0);
-      L.vs[r] = __builtin_amdgcn_raw_buffer_load_b16(P.vs8, soff8, so, 0);
+  for (int i = 0; i < kPairs; ++i) {
+    uint32_t e8 = e[i], e4 = e[i];
+    if constexpr (TIERS == kRowsMixed) {
+      const bool hot = (e[i] >> 30) == 1u;
+      e8 = hot ? e[i] ^ kHotBit : kNoRow;
+      e4 = hot ? kNoRow : e[i];
+    }
+    if constexpr (TIERS != kRowsInt4) {
+      R.w8[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r8, (int)(e8 * 256u + 8u * g), 0, 0));
+      R.s8[i] = __builtin_amdgcn_raw_buffer_load_b16(rs8, (int)(e8 * kSh8 + 2u * ((8u * g) / G8)), 0, 0);
+    }
+    if constexpr (TIERS != kRowsInt8) {
+      R.w4[i] = __builtin_amdgcn_raw_buffer_load_b32(r4, (int)(e4 * 128u + 4u * g), 0, 0);
+      R.s4[i] = __builtin_amdgcn_raw_buffer_load_b16(rs4, (int)(e4 * 16u + 2u * (g >> 2)), 0, 0);
+    }
+  }
+}
+
+// Dequantize the tile into the wavefront's LDS rows (row-major, 16 bytes per lane); sm_row: the head's 256 smoothing
+// factors in LDS.
+template <int TIERS, bool SM>
+KVT_DEV void store_rows(const Raw& R, const uint32_t e[kPairs], uint16_t* kt, int lane, const uint16_t* sm_row) {
+  uint4 sm{};
+  if constexpr (SM) sm = *reinterpret_cast<const uint4*>(&sm_row[8 * (lane & 31)]);
+  uint16_t* dst = &kt[(lane >> 5) * kKPitch + 8 * (lane & 31)];
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) {
+    uint32_t m[4];
+    uint32_t sb;
+    float off;
+    if constexpr (TIERS == kRowsInt8) {
+      magic8(R.w8[i], m);
+      sb = R.s8[i], off = 1152.0f;
+    } else if constexpr (TIERS == kRowsInt4) {
+      magic4(R.w4[i], m);
+      sb = R.s4[i], off = 1032.0f;
     } else {
-      L.kw[r] = __builtin_amdgcn_raw_buffer_load_b32(P.k4, off4, co, 0);
-      L.vw[r] = __builtin_amdgcn_raw_buffer_load_b32(P.v4, off4, co, 0);
-      L.ks[r] = __builtin_amdgcn_raw_buffer_load_b16(P.ks4, soff4, so, 0);
-      L.vs[r] = __builtin_amdgcn_raw_buffer_load_b16(P.vs4, soff4, so, 0);
-    }
-  }
-}
-
-// A tile's 16 columns resolved by lanes 0-15 (lane r: column c0 + r): attended or not, tier, and the row's byte
-// offsets in its tier (codes: INT8 rows D bytes, INT4 rows D / 2; scales).
-struct TileCols {
-  int flags;   // bit 0 attended, bit 1 ring (INT8) row
-  uint32_t coff, soff;
-};
-
-// Resolve a tile's columns: position from the index row, slot from req_to_token, tier from the owner table (three
-// dependent loads, independent of Q).
-template <int KIND, int G8>
-KVT_DEV TileCols resolve_tile(const SparseArgs& A, int64_t c0, int64_t c_end, const int32_t* idx_row, int64_t L,
-                              int64_t req, int h, int lane) {
-  const int64_t col = c0 + (lane & 15);
-  bool valid = false, hot = KIND == 0;
-  int64_t row = 0;
-  if (lane < kRows && col < c_end) {
-    const int64_t pos = idx_row[col * A.si_n];
-    if (pos >= 0 && pos < L) {
-      valid = true;
-      const int64_t slot = A.req_to_token[req * A.req_stride + pos];
-      row = slot;
-      if constexpr (KIND == 2) {
-        const int64_t r = slot & A.ring_mask;
-        if ((int64_t)A.owner[r] == slot) {
-          hot = true;
-          row = r;
-        }
-      }
-    }
-  }
-  const int64_t rh = row * A.H + h;
-  TileCols tc;
-  tc.flags = (valid ? 1 : 0) | (hot ? 2 : 0);
-  tc.coff = !valid ? kNoRow : (uint32_t)(hot ? rh * kD : rh * (kD / 2));
-  tc.soff = !valid ? kNoRow : (uint32_t)(hot ? rh * (kD / G8) * 2 : rh * (kD / kG4) * 2);
-  return tc;
-}
-
-// One resolved 16-column tile of a wavefront, folded into its running softmax state (m, l per q head n16 of this
-// lane, o): load and dequantize K into the wavefront's LDS rows, S^T = K Q^T, dequantize V into the same rows,
-// online softmax, O += P V.
-// hook(k) runs other work at three points: k = 0 before the tile's loads, 1 after its K rows are in LDS, 2 after
-// S^T.
-template <int KIND, int G8, int TIERS, typename Hook>
-KVT_DEV void attend_tile(const SparseArgs& A, const PoolRsrc& P, const uint16_t* qs, uint16_t* kt, const TileCols& tc,
-                         int lane, const float smk[4], const float smv[4], float& m_run, float& l_run, f4 o[16],
-                         Hook&& hook) {
-  const int n16 = lane & 15, kq = lane >> 4;
-  const int flags = tc.flags;
-  TileLoads T;
-  hook(0);
-  issue_tile<G8, TIERS>(P, flags, tc.coff, tc.soff, lane, T);
-
-  // K rows into this wavefront's LDS rows (row-major); a wavefront's LDS accesses complete in order, so these
-  // stores land after the previous tile's V reads
+      uint32_t m8[4];
+      magic8(R.w8[i], m8);
+      magic4_as8(R.w4[i], m);
+      const bool hot = (e[i] >> 30) == 1u;
 #pragma unroll
-  for (int r = 0; r < kRows; ++r)
-    *reinterpret_cast<uint2*>(&kt[r * kKPitch + 4 * lane]) = dequant4((T.fl[r] & 2) != 0, T.kw[r], T.ks[r], lane, smk);
-  hook(1);
+      for (int j = 0; j < 4; ++j) m[j] = hot ? m8[j] : m[j];
+      sb = hot ? R.s8[i] : R.s4[i];
+      off = hot ? 1152.0f : 1032.0f;
+    }
+    *reinterpret_cast<uint4*>(dst + 2 * i * kKPitch) = rows_bf16<SM, TIERS == kRowsInt4>(m, sb, off, sm);
+  }
+}
+
+// One resolved 16-column tile of a wavefront, whose raw rows are K and V, folded into its running softmax state (m, l
+// per q head n16 of this lane, o): dequantize K into the wavefront's LDS rows, S^T = K Q^T, dequantize V into the same
+// rows, online softmax, O += P V.  e: the row words of this lane's half; vm: bit r set when row r is attended
+// (wave-uniform).  NEXT: K and V are loaded again, for the tile whose words are en, as soon as their registers are
+// free, so that those loads travel beside this tile's work.
+template <int G8, int TIERS, bool SM, bool NEXT>
+KVT_DEV void attend_tile(const SparseArgs& A, const PoolRsrc& P, const bf8 qop[8], uint16_t* kt,
+                         Raw& K, Raw& V, const uint32_t e[kPairs], uint32_t vm, const uint32_t en[kPairs], int lane,
+                         const uint16_t* sm, float& m_run, float& l_run, f4 o[16]) {
+  const int n16 = lane & 15, kq = lane >> 4;
+  // K rows into this wavefront's LDS rows; a wavefront's LDS accesses complete in order, so these stores land after
+  // the previous tile's V reads
+  store_rows<TIERS, SM>(K, e, kt, lane, sm);
+  if constexpr (NEXT) issue_rows<G8, TIERS>(P.k8, P.ks8, P.k4, P.ks4, en, lane, K);
+  __builtin_amdgcn_sched_barrier(0);
   // S^T = K Q^T: lane l holds rows 4 (l >> 4) + i of q head l & 15
   f4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const uint2 ka = *reinterpret_cast<const uint2*>(&kt[n16 * kKPitch + 16 * k + 4 * kq]);
-    const uint2 qb = *reinterpret_cast<const uint2*>(&qs[n16 * kKPitch + 16 * k + 4 * kq]);
-    s = mfma_bf16(__builtin_bit_cast(bf4, ka), __builtin_bit_cast(bf4, qb), s);
+  for (int k = 0; k < 8; ++k) {
+    const uint4 ka = *reinterpret_cast<const uint4*>(&kt[n16 * kKPitch + 32 * k + 8 * kq]);
+    s = mfma_bf16(__builtin_bit_cast(bf8, ka), qop[k], s);
   }
-  hook(2);
+  __builtin_amdgcn_sched_barrier(0);
   // from here to P the tile's chain runs at a raised wave priority: the V rows and the softmax issue ahead of the
   // other wavefronts' work on the SIMD, which keeps the products that wait for them fed (slot-pool decode and the
   // paged prefix-chunk attention ~6 % faster than without)
   __builtin_amdgcn_s_setprio(1);
   // V rows into the same LDS rows (the stores stay behind the K reads above, which may alias them)
-#pragma unroll
-  for (int r = 0; r < kRows; ++r)
-    *reinterpret_cast<uint2*>(&kt[r * kKPitch + 4 * lane]) = dequant4((T.fl[r] & 2) != 0, T.vw[r], T.vs[r], lane, smv);
+  store_rows<TIERS, SM>(V, e, kt, lane, sm + kD);
+  if constexpr (NEXT) issue_rows<G8, TIERS>(P.v8, P.vs8, P.v4, P.vs4, en, lane, V);
   // online softmax (log2 units): rows 4 kq + i of this lane's head, the other 12 rows in lanes n16 + 16 j
   constexpr float kLog2e = 1.4426950408889634f;
   const float cs = A.scale * kLog2e;
   float tv[4], mloc = -INFINITY;
+  const uint32_t vq = vm >> (4 * kq);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int f = __shfl(flags, 4 * kq + i, 64);   // the row's resolve lane
-    tv[i] = (f & 1) ? s[i] * cs : -INFINITY;
+    tv[i] = ((vq >> i) & 1u) != 0 ? s[i] * cs : -INFINITY;
     mloc = fmaxf(mloc, tv[i]);
   }
   const float m_new = fmaxf(m_run, max_xor16_32(mloc));
@@ -302,7 +321,9 @@ KVT_DEV void attend_tile(const SparseArgs& A, const PoolRsrc& P, const uint16_t*
   float p[4], lsum = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    p[i] = m_new == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(tv[i] - m_new);
+    // (the exponent in one rounding of the difference: the rounded score tv alone is off by up to 2^-24 |tv|)
+    const float d = fmaf(s[i], cs, -m_new);
+    p[i] = tv[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(d);
     lsum += p[i];
   }
   l_run = l_run * alpha + sum_xor16_32(lsum);
@@ -317,13 +338,14 @@ KVT_DEV void attend_tile(const SparseArgs& A, const PoolRsrc& P, const uint16_t*
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[n][i] *= ai[i];
   }
-  // P as bf16 high part + bf16 remainder (two products per step): P keeps ~16 significant bits, against 8 for a
-  // plain bf16 cast, so a peaked softmax stays within the fp32 reference's tolerance
+  // P as bf16 high part + bf16 remainder: P keeps ~16 significant bits, against 8 for a plain bf16 cast, so a peaked
+  // softmax stays within the fp32 reference's tolerance.  Both go through one 32-deep product: this lane's 8 k indices
+  // are the high parts of its 4 rows and their remainders, against the same 4 V rows twice (a 16x16x32 product takes
+  // the matrix pipe as long as a 16x16x16 one).
   const uint32_t h01 = bf16x2(p[0], p[1]), h23 = bf16x2(p[2], p[3]);
   const uint32_t l01 = bf16x2(p[0] - __uint_as_float(h01 << 16), p[1] - __uint_as_float(h01 & 0xffff0000u));
   const uint32_t l23 = bf16x2(p[2] - __uint_as_float(h23 << 16), p[3] - __uint_as_float(h23 & 0xffff0000u));
-  const bf4 pa = __builtin_bit_cast(bf4, uint2{h01, h23});
-  const bf4 pb = __builtin_bit_cast(bf4, uint2{l01, l23});
+  const bf8 pa = __builtin_bit_cast(bf8, uint4{h01, h23, l01, l23});
   __builtin_amdgcn_s_setprio(0);
   // O = P V.  B = V[rows 4 kq + k][channel 16 n + n16] by the transposing read: in each 16-lane group, lane L's
   // element k comes from element L & 3 of the 8 bytes lane 4 k + (L >> 2) addresses, so lane m addresses
@@ -331,29 +353,70 @@ KVT_DEV void attend_tile(const SparseArgs& A, const PoolRsrc& P, const uint16_t*
   const uint32_t vbase = (uint32_t)(uintptr_t)&kt[(4 * kq + (n16 >> 2)) * kKPitch + 4 * (n16 & 3)];
 #pragma unroll
   for (int n = 0; n < 16; ++n) {
-    const bf4 vop = __builtin_bit_cast(
-        bf4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vbase + 32u * (uint32_t)n)));
-    o[n] = mfma_bf16(pb, vop, mfma_bf16(pa, vop, o[n]));
+    const uint2 v = __builtin_bit_cast(
+        uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vbase + 32u * (uint32_t)n)));
+    o[n] = mfma_bf16(pa, __builtin_bit_cast(bf8, uint4{v.x, v.y, v.x, v.y}), o[n]);
+    if ((n & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // (at most 4 V operands held at once)
   }
 }
 
-// A tile through the body for its rows' tiers: single-tier pools know them; in the tiered pool a tile whose 16 rows
-// all sit in one tier (most of them: the ring holds a small share of the slots) takes a body without a branch per row.
-template <int KIND, int G8, typename Hook>
-KVT_DEV void attend_tile_any(const SparseArgs& A, const PoolRsrc& P, const uint16_t* qs, uint16_t* kt,
-                             const TileCols& tc, int lane, const float smk[4], const float smv[4], float& m_run,
-                             float& l_run, f4 o[16], Hook&& hook) {
+template <int N>
+struct Tiers {
+  static constexpr int value = N;
+};
+
+// The tile of a one-tile decode block through the body for its rows' tiers: single-tier pools know them; in the
+// tiered pool a tile whose 16 rows all sit in one tier (most of them: the ring holds a small share of the slots) takes
+// that tier's body.  Lane r < 16 holds row r's word.
+template <int KIND, int G8, bool SM>
+KVT_DEV void attend_tile_any(const SparseArgs& A, const PoolRsrc& P, const bf8 qop[8], uint16_t* kt, uint32_t word,
+                             int lane, const uint16_t* sm, float& m_run, float& l_run, f4 o[16]) {
+  const uint32_t vm = (uint32_t)__builtin_amdgcn_ballot_w64(word != kNoRow) & 0xffffu;
+  uint32_t e[kPairs];
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) e[i] = (uint32_t)__shfl((int)word, 2 * i + (lane >> 5), 64);
+  auto one = [&](auto tiers) {
+    constexpr int T = decltype(tiers)::value;
+    Raw K, V;
+    issue_rows<G8, T>(P.k8, P.ks8, P.k4, P.ks4, e, lane, K);
+    issue_rows<G8, T>(P.v8, P.vs8, P.v4, P.vs4, e, lane, V);
+    attend_tile<G8, T, SM, false>(A, P, qop, kt, K, V, e, vm, e, lane, sm, m_run, l_run, o);
+  };
   if constexpr (KIND != 2) {
-    attend_tile<KIND, G8, KIND == 0 ? kRowsInt8 : kRowsInt4>(A, P, qs, kt, tc, lane, smk, smv, m_run, l_run, o, hook);
+    one(Tiers<KIND == 0 ? kRowsInt8 : kRowsInt4>{});
   } else {
-    const uint64_t hot = __builtin_amdgcn_ballot_w64((tc.flags & 2) != 0) & 0xffffu;
-    if (hot == 0)
-      attend_tile<KIND, G8, kRowsInt4>(A, P, qs, kt, tc, lane, smk, smv, m_run, l_run, o, hook);
-    else if (hot == 0xffffu)
-      attend_tile<KIND, G8, kRowsInt8>(A, P, qs, kt, tc, lane, smk, smv, m_run, l_run, o, hook);
-    else
-      attend_tile<KIND, G8, kRowsMixed>(A, P, qs, kt, tc, lane, smk, smv, m_run, l_run, o, hook);
+    const uint32_t hot = (uint32_t)__builtin_amdgcn_ballot_w64((word >> 30) == 1u) & 0xffffu;
+    if (hot == 0) {
+      one(Tiers<kRowsInt4>{});
+    } else if (hot == vm) {
+#pragma unroll
+      for (int i = 0; i < kPairs; ++i) e[i] = e[i] == kNoRow ? kNoRow : e[i] ^ kHotBit;
+      one(Tiers<kRowsInt8>{});
+    } else {
+      one(Tiers<kRowsMixed>{});
+    }
   }
+}
+
+// Resolve a tile's columns, lane r < 16 column c0 + r, into its row word: position from the index row, slot from
+// req_to_token, tier from the owner table (three dependent loads, independent of Q).
+template <int KIND>
+KVT_DEV uint32_t resolve_tile(const SparseArgs& A, int64_t c0, int64_t c_end, const int32_t* idx_row, int64_t L,
+                              int64_t req, int h, int lane) {
+  const int64_t col = c0 + (lane & 15);
+  uint32_t word = kNoRow;
+  if (lane < kRows && col < c_end) {
+    const int64_t pos = idx_row[col * A.si_n];
+    if (pos >= 0 && pos < L) {
+      const int64_t slot = A.req_to_token[req * A.req_stride + pos];
+      word = (uint32_t)(slot * A.H + h);
+      if constexpr (KIND == 2) {
+        const int64_t r = slot & A.ring_mask;
+        if ((int64_t)A.owner[r] == slot) word = (uint32_t)(r * A.H + h) | kHotBit;
+      }
+    }
+  }
+  return word;
 }
 
 // LDS of a block: one tile buffer per wavefront (K rows until S is formed, then V rows; 42 KB per block), after the
@@ -362,25 +425,32 @@ template <int CAP>
 struct BlockLds {
   uint16_t kv[kWaves][kRows * kKPitch];
   uint16_t qs[kHeads * kKPitch];
-  uint2 cols[CAP];             // prefill rows: the query's resolved columns, ring rows first and INT4 rows last
+  uint16_t sm[2 * kD];         // smoothing factors (fp16) of K, then V; read when they are not all 1
+  uint32_t cols[CAP + 3 * kRows];   // the resolved columns' row words: ring rows first, INT4 rows from entry
+                                    // CAP + 2 kRows down, each part padded with kNoRow to whole tiles; then one
+                                    // tile of kNoRow
   int counts[2 * kWaves];
+  int ones[kWaves];            // wavefront w's smoothing factors are all 1
   int last;                    // decode merged in the launch: this block counted last for its (request, KV head)
 };
 constexpr int kRowCols = 4096;   // prefill rows: selected columns resolved per pass (74 KB of LDS per block)
 constexpr int kMultiCols = 1024; // decode blocks of several tiles per wavefront (50 KB of LDS per block)
 
-// The selected columns [k0, k1) (at most kRowCols) of a prefill block's query row, resolved by all its threads
-// together into the column table and partitioned by tier: ring (INT8) rows to cols[0 .. nh), INT4 rows to
-// cols[CAP - nc .. CAP) (from the end), unattended columns dropped (patches/kv_paged_prefix.py:199-229: position in
+// The selected columns [k0, k1) (at most CAP) of a block's query row, resolved by all its threads
+// together into the column table and partitioned by tier: ring (INT8) rows to cols[0 .. nh), INT4 rows from the end
+// of the table down, both padded with kNoRow to whole tiles, unattended columns dropped (patches/kv_paged_prefix.py:199-229: position in
 // [0, L)).  J columns per thread, so the position, slot and owner loads of many columns are in flight at once; a
 // block scan of the per-thread counts places them, in an order fixed by the columns (thread, then j), so the result
 // does not depend on timing.  Every tile of 16 table entries then sits in one tier.
-template <int KIND, int G8, int CAP, int J>
+template <int KIND, int CAP, int J>
 KVT_DEV void resolve_rows(const SparseArgs& A, int64_t k0, int64_t k1, const int32_t* idx_row, int64_t L,
                           int64_t req, int h, BlockLds<CAP>& S, int& nh, int& nc) {
   constexpr int kThreads = 64 * kWaves;
   static_assert(J * kThreads >= CAP, "a pass covers the table");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kEnd = CAP + 2 * kRows - 1;   // nh + nc <= CAP: the parts and their padding never meet
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (a later pass's column numbers are formed there, not held across the tile loops)
+  const int lane = tid & 63, wave = tid >> 6;
   const int32_t* r2t = A.req_to_token + req * A.req_stride;
   int pos[J], slot[J], own[J];
   bool live[J];
@@ -421,36 +491,41 @@ KVT_DEV void resolve_rows(const SparseArgs& A, int64_t k0, int64_t k1, const int
     if (w < wave) oh += a, oc += c;
     nh += a, nc += c;
   }
+  nh = __builtin_amdgcn_readfirstlane(nh), nc = __builtin_amdgcn_readfirstlane(nc);   // (the same in every lane)
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     if (!live[j]) continue;
     const int64_t row = hot[j] && KIND == 2 ? ((int64_t)slot[j] & A.ring_mask) : (int64_t)slot[j];
-    const int64_t rh = row * A.H + h;
-    const uint2 e = hot[j] ? uint2{(uint32_t)(rh * kD), (uint32_t)(rh * (kD / G8) * 2)}
-                           : uint2{(uint32_t)(rh * (kD / 2)), (uint32_t)(rh * (kD / kG4) * 2)};
+    const uint32_t word = (uint32_t)(row * A.H + h);
     if (hot[j])
-      S.cols[oh++] = e;
+      S.cols[oh++] = word;
     else
-      S.cols[CAP - 1 - oc++] = e;
+      S.cols[kEnd - oc++] = word;
+  }
+  if (tid < kRows) {
+    if (nh + tid < (nh + kRows - 1) / kRows * kRows) S.cols[nh + tid] = kNoRow;
+    if (nc + tid < (nc + kRows - 1) / kRows * kRows) S.cols[kEnd - nc - tid] = kNoRow;
+    S.cols[kEnd + 1 + tid] = kNoRow;
   }
 }
 
-// Tile t of a partitioned table: hot tiles 0 .. ceil(nh / 16) - 1 read entries 16 t .. from the front, the INT4
-// tiles after them entries from the end; lane r < 16 takes one entry (past the part's count: not attended).
-template <int CAP>
-KVT_DEV TileCols table_tile(const BlockLds<CAP>& S, int t, int th, int nh, int nc, int lane) {
-  const int r = lane & 15;
-  const bool hot = t < th;
-  const int i = hot ? 16 * t + r : 16 * (t - th) + r;
-  const bool ok = lane < kRows && i < (hot ? nh : nc);
-  TileCols x;
-  x.flags = ok ? (hot ? 3 : 1) : 0;
-  x.coff = kNoRow, x.soff = kNoRow;
-  if (ok) {
-    const uint2 e = S.cols[hot ? i : CAP - 1 - i];
-    x.coff = e.x, x.soff = e.y;
-  }
-  return x;
+// The row words of tile t < nt of a part of the table (HOT: from the front, INT4: from the end), for this lane's
+// half; t >= nt: a tile of kNoRow words, whose loads cost no traffic.
+template <bool HOT, int CAP>
+KVT_DEV void table_tile(const BlockLds<CAP>& S, int t, int nt, int lane, uint32_t e[kPairs]) {
+  const int i0 = 16 * t;
+  const int lo = t >= nt ? CAP + 2 * kRows : HOT ? i0 : CAP + kRows - i0;   // the tile's lowest table entry
+  // (ascending for either part: the order of rows within a tile is of no consequence, the padding's place is)
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) e[i] = S.cols[lo + 2 * i + (lane >> 5)];
+}
+
+// The attended rows of tile t of a part of n entries: its first n - 16 t words, the last ones in the INT4 part's
+// descending order.
+template <bool HOT>
+KVT_DEV uint32_t table_mask(int t, int n) {
+  const int rem = n - 16 * t;
+  return rem >= kRows ? 0xffffu : HOT ? (1u << rem) - 1u : (0xffffu << (kRows - rem)) & 0xffffu;
 }
 
 // Device-scope stores and loads of the split partials: the partials cross XCDs (each has its own L2), so they are
@@ -601,6 +676,11 @@ KVT_DEV PoolRsrc tier_rsrc(const SparseArgs& A, int H) {
   return P;
 }
 
+template <bool B>
+struct Flag {
+  static constexpr bool value = B;
+};
+
 // ROWS: prefill rows (one query row per block) instead of decode splits; MULTI: a decode block of several tiles per
 // wavefront; CAP > 1: the block resolves its columns into a column table of CAP entries partitioned by tier first.
 template <int KIND, int G8, bool ROWS, bool MULTI, int CAP>
@@ -635,12 +715,10 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     }
   };
   if constexpr (!ROWS) load_q(b);
-  // smoothing factors of this lane's channels 4 lane .. 4 lane + 3 (an absent factor: an empty buffer, read as 0)
-  const uint32_t smb = (uint32_t)H * kD * 2;
-  const uint2 wsk = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(
-                                                  rsrc(A.sm_k, A.sm_k != nullptr ? smb : 0u), (h * kD + 4 * lane) * 2, 0, 0));
-  const uint2 wsv = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(
-                                                  rsrc(A.sm_v, A.sm_v != nullptr ? smb : 0u), (h * kD + 4 * lane) * 2, 0, 0));
+  // the head's smoothing factors, 2 per thread: K's, then V's (an absent tensor: all 1)
+  const uint16_t* smp = threadIdx.x < kD / 2 ? A.sm_k : A.sm_v;
+  const uint32_t smw = smp != nullptr ? reinterpret_cast<const uint32_t*>(smp + h * kD)[threadIdx.x & (kD / 2 - 1)]
+                                      : 0x3c003c00u;
   __builtin_amdgcn_sched_barrier(0);
   const int64_t req = idx_value(wreq), x0 = idx_value(w0), x1 = idx_value(w1), L = len;
   // the block's query row and column range
@@ -668,14 +746,14 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
   asm volatile("" ::"s"(idx_row), "s"(L), "s"(req), "s"(c_end), "s"(A.req_to_token), "s"(A.req_stride),
                "s"(A.owner), "s"(A.ring_mask), "s"(A.si_n));
   // the wavefront's first tile (prefill rows: the first pass of the column table)
-  TileCols tc0{};
+  uint32_t word0 = kNoRow;
   const bool has_tile = c_begin + kRows * wave < c_end;
   int nh = 0, nc = 0;
   if constexpr (CAP > 1)
-    resolve_rows<KIND, G8, CAP, CAP / (64 * kWaves)>(A, c_begin, c_begin + CAP < c_end ? c_begin + CAP : c_end, idx_row,
+    resolve_rows<KIND, CAP, CAP / (64 * kWaves)>(A, c_begin, c_begin + CAP < c_end ? c_begin + CAP : c_end, idx_row,
                                                      L, req, h, S, nh, nc);
   else if (has_tile)
-    tc0 = resolve_tile<KIND, G8>(A, c_begin + kRows * wave, c_end, idx_row, L, req, h, lane);
+    word0 = resolve_tile<KIND>(A, c_begin + kRows * wave, c_end, idx_row, L, req, h, lane);
 #pragma unroll
   for (int k = 0; k < kQChunks; ++k) {
     const int i = (int)threadIdx.x + 64 * kWaves * k;
@@ -695,45 +773,68 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     P.ks4 = rsrc(A.ks, KIND == 0 ? 0u : s4);
     P.vs4 = rsrc(A.vs, KIND == 0 ? 0u : s4);
   }
-  float smk[4], smv[4];
-  const uint32_t swk[4] = {wsk.x, wsk.x >> 16, wsk.y, wsk.y >> 16}, swv[4] = {wsv.x, wsv.x >> 16, wsv.y, wsv.y >> 16};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    smk[i] = A.sm_k != nullptr ? f16_bits_to_f32((uint16_t)swk[i]) : 1.f;
-    smv[i] = A.sm_v != nullptr ? f16_bits_to_f32((uint16_t)swv[i]) : 1.f;
-  }
+  reinterpret_cast<uint32_t*>(S.sm)[threadIdx.x] = smw;
+  const bool ones = __all(smw == 0x3c003c00u);
+  if (lane == 0) S.ones[wave] = ones;
   __syncthreads();   // q staged
+  // every factor of the head 1: the bodies without the products
+  const bool identity = __builtin_amdgcn_readfirstlane(S.ones[0] & S.ones[1] & S.ones[2] & S.ones[3]) != 0;
+
+  // the B operands of the score products: channels 32 k + 8 (lane >> 4) .. + 7 of q head lane & 15
+  bf8 qop[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    qop[k] = __builtin_bit_cast(bf8, *reinterpret_cast<const uint4*>(&qs[(lane & 15) * kKPitch + 32 * k + 8 * (lane >> 4)]));
 
   float m_run = -INFINITY, l_run = 0.f;   // of q head lane & 15
   f4 o[16];                               // O[head 4 (lane >> 4) + i][channel 16 n + (lane & 15)]
 #pragma unroll
   for (int n = 0; n < 16; ++n) o[n] = f4{0.f, 0.f, 0.f, 0.f};
   if constexpr (CAP > 1) {
-    // passes of the column table (the first resolved above): wavefront w takes tiles w, w + 4, ..., ring tiles first
-    for (int64_t k0 = c_begin; k0 < c_end; k0 += CAP) {
-      const int64_t k1 = k0 + CAP < c_end ? k0 + CAP : c_end;
-      if (k0 > c_begin) {
-        __syncthreads();   // the previous pass's entries are read
-        resolve_rows<KIND, G8, CAP, CAP / (64 * kWaves)>(A, k0, k1, idx_row, L, req, h, S, nh, nc);
-        __syncthreads();
+    // passes of the column table (the first resolved above): wavefront w takes tiles w, w + 4, ..., ring tiles first.
+    // The choice by the smoothing factors stands outside the passes: inside, the two bodies' accumulators were held
+    // in separate registers.
+    auto passes = [&](auto smooth) {
+      constexpr bool SM = decltype(smooth)::value;
+      for (int64_t k0 = c_begin; k0 < c_end; k0 += CAP) {
+        const int64_t k1 = k0 + CAP < c_end ? k0 + CAP : c_end;
+        if (k0 > c_begin) {
+          __syncthreads();   // the previous pass's entries are read
+          resolve_rows<KIND, CAP, CAP / (64 * kWaves)>(A, k0, k1, idx_row, L, req, h, S, nh, nc);
+          __syncthreads();
+        }
+        const int th = (nh + kRows - 1) / kRows, nt = th + (nc + kRows - 1) / kRows;
+        int t = wave;
+        // the tiles t, t + kWaves, .. < t_end of one tier (t0: its first tile, n: its entries)
+        auto run = [&](const PoolRsrc& R, auto hot, int t0, int t_end, int n) {
+          constexpr bool HOT = decltype(hot)::value;
+          constexpr int T = HOT ? kRowsInt8 : kRowsInt4;
+          if (t >= t_end) return;
+          uint32_t e[kPairs];
+          Raw K, V;
+          table_tile<HOT>(S, t - t0, t_end - t0, lane, e);
+          issue_rows<G8, T>(R.k8, R.ks8, R.k4, R.ks4, e, lane, K);
+          issue_rows<G8, T>(R.v8, R.vs8, R.v4, R.vs4, e, lane, V);
+          for (; t < t_end; t += kWaves) {
+            table_tile<HOT>(S, t + kWaves - t0, t_end - t0, lane, e);
+            attend_tile<G8, T, SM, true>(A, R, qop, kv[wave], K, V, e, table_mask<HOT>(t - t0, n), e, lane, S.sm, m_run,
+                                         l_run, o);
+          }
+        };
+        // the ring (INT8) tiles, then the INT4 ones, each tier's descriptors in turn
+        if constexpr (KIND != 1) run(tier_rsrc<KIND, G8, true>(A, H), Flag<true>{}, 0, th, nh);
+        if constexpr (KIND != 0) run(tier_rsrc<KIND, G8, false>(A, H), Flag<false>{}, th, nt, nc);
       }
-      const int th = (nh + kRows - 1) / kRows, nt = th + (nc + kRows - 1) / kRows;
-      int t = wave;
-      if constexpr (KIND != 1) {   // the ring (INT8) tiles, then the INT4 ones, each tier's descriptors in turn
-        const PoolRsrc P8 = tier_rsrc<KIND, G8, true>(A, H);
-        for (; t < th; t += kWaves)
-          attend_tile<KIND, G8, kRowsInt8>(A, P8, qs, kv[wave], table_tile(S, t, th, nh, nc, lane), lane, smk, smv,
-                                           m_run, l_run, o, [](int) {});
-      }
-      if constexpr (KIND != 0) {
-        const PoolRsrc P4 = tier_rsrc<KIND, G8, false>(A, H);
-        for (; t < nt; t += kWaves)
-          attend_tile<KIND, G8, kRowsInt4>(A, P4, qs, kv[wave], table_tile(S, t, th, nh, nc, lane), lane, smk, smv,
-                                           m_run, l_run, o, [](int) {});
-      }
-    }
-  } else {   // at most one tile per wavefront (64 columns per block): no state is live across its loads
-    if (has_tile) attend_tile_any<KIND, G8>(A, P, qs, kv[wave], tc0, lane, smk, smv, m_run, l_run, o, [](int) {});
+    };
+    if (identity)
+      passes(Flag<false>{});
+    else
+      passes(Flag<true>{});
+  } else if (has_tile) {   // at most one tile per wavefront (64 columns per block): no state is live across its loads
+    if (identity)
+      attend_tile_any<KIND, G8, false>(A, P, qop, kv[wave], word0, lane, S.sm, m_run, l_run, o);
+    else
+      attend_tile_any<KIND, G8, true>(A, P, qop, kv[wave], word0, lane, S.sm, m_run, l_run, o);
   }
 
   // merge the 4 wavefronts through LDS, 8 q heads per pass: wavefront w stores the O rows of the pass's heads and
@@ -825,7 +926,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 }
 
 // decode of long selections: the block's 64 A.tiles columns resolved into its column table, a wavefront looping over
-// its tiles with the accumulators live; 2 blocks per CU
+// its tiles with the accumulators and the next tile's rows live; 2 blocks per CU (held to the 168 registers of 3, the
+// next tile's loads and the operand reads no longer overlap: 74 us against 55 us)
 template <int KIND, int G8>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2)))
 sparse_decode_multi_kernel(SparseArgs A) {
@@ -847,10 +949,10 @@ int pool_args(int kind, int64_t pool_rows, const void* ring_k, const void* owner
   if (H <= 0 || Hq % H != 0 || Hq / H > kHeads || D != kD || kind < 0 || kind > 2) return KVT_EINVAL;
   if (kind == 2 && (owner == nullptr || ring_k == nullptr || ((ring_mask + 1) & ring_mask) != 0)) return KVT_EINVAL;
   if (pool_rows <= 0 || (kind != 1 && group8 != 64 && group8 != 256)) return KVT_EINVAL;
-  // byte offsets are 32-bit and must stay below kNoRow (rows * H * D bytes of INT8 codes, / 2 for INT4)
+  // byte offsets are 32-bit and must stay below 2^31 (rows * H * D bytes of INT8 codes, / 2 for INT4)
   *rows8 = kind == 2 ? ring_mask + 1 : (kind == 0 ? pool_rows : 0);
   *rows4 = kind == 0 ? 0 : pool_rows;
-  if (*rows8 * H * kD >= (int64_t)kNoRow || *rows4 * H * (kD / 2) >= (int64_t)kNoRow) return KVT_ERANGE;
+  if (*rows8 * H * kD >= (1ll << 31) || *rows4 * H * (kD / 2) >= (1ll << 31)) return KVT_ERANGE;
   return KVT_OK;
 }
 

@@ -216,7 +216,7 @@ def qwen_sparse_kv_extraction_compact_triton(
               out_v.data_ptr(), _lib.stream())
 
 
-_MULTI_BLOCKS = 768   # blocks of a long-selection launch: one per resident slot, 3 per CU (50 KB of LDS, <= 168 VGPRs)
+_MULTI_BLOCKS = 512   # blocks of a long-selection launch: one per resident slot, 2 per CU (256 VGPRs)
 
 
 def qwen_sparse_decode_attn(
@@ -276,7 +276,8 @@ def qwen_sparse_decode_attn(
     _lib.require_device(q, k, v, req_to_token, indices, out)
     scale = float(dim ** -0.5) if scale is None else float(scale)
     # blocks of 64 selected columns (a 16-column tile per wavefront) while the launch holds at most 1,024 of them;
-    # longer selections take `tiles` tiles per wavefront in about one block per resident slot (3 per CU), each
+    # longer selections take `tiles` tiles per wavefront in about one block per resident slot (2 per CU: 55 us
+    # for 4 x 65,536 dense positions, against 63 us at 1,024 blocks and 80 us at 768), each
     # partial then covering 64 x tiles columns
     tiles64 = (int(topk) + 63) // 64
     blocks = batch * heads * tiles64
