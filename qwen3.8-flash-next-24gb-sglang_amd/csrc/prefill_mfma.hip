@@ -5,9 +5,11 @@
 // values come from the cache tiers (INT4 pages below hot_start, INT8 ring above) or, for a chunk without a prefix,
 // from the chunk's own bf16 K/V (the reference attends to fresh bf16 K/V there).
 //
-// Work item = (sequence, KV head, tile of queries), 8 wavefronts (2 per SIMD), heaviest (latest) query tiles
-// first.  A wavefront owns 16 query rows = 16 / gs queries x the gs q heads of the KV head (gs <= 16; rows beyond
-// 16 / gs * gs idle).  The block walks the keys in tiles of 32 positions.  All 512 threads dequantize a tile ONCE
+// Work item = (sequence, KV head, tile of 128 query rows), 8 wavefronts (2 per SIMD), heaviest (latest) query tiles
+// first.  The query rows of a KV head are its (query, q head) pairs in that order, row = query * gs + head (gs <= 16 q
+// heads per KV head); a tile takes 128 of them and a wavefront 16, whatever query they fall in, so that no matrix row
+// idles where gs does not divide 16 (24 / 2 heads: 12 of 16 rows in use when a wavefront took whole queries, 4,096
+// queries over their own keys 358 -> 282 us).  The block walks the keys in tiles of 32 positions.  All 512 threads dequantize a tile ONCE
 // into LDS (each thread 16 channels of a K row and 8 channels of two V rows), with the next tile's codes already
 // loaded into registers during the matrix work on the current one; the eight wavefronts then reuse it for their
 // 16 rows each (dequantizing per query row is what made the reference's fused kernel slow,
@@ -562,14 +564,17 @@ KVT_DEV void v_step(int j, const RawV& x, uint32_t a[4], uint32_t b[4], uint8_t*
 }
 
 constexpr int kAheadK = 2, kAheadV = 4;   // LDS operand reads issued this many matrix steps ahead
-constexpr int kWaves = 8;               // 2 per SIMD: each wavefront 16 rows (16 / gs queries x gs heads)
+constexpr int kWaves = 8;               // 2 per SIMD: each wavefront 16 rows
 
-// The queries of one query tile (qb queries of sequence b) and the keys they see.
+constexpr int kTileRows = 16 * kWaves;  // query rows of a query tile
+
+// The queries of one query tile (rows 128 qt .. 128 qt + 127 of a KV head of sequence b) and the keys they see.
 struct QTile {
   int64_t qs, q_len, L, q_pos0, qt0, key_end;
+  int rem;      // head of the tile's first row (the row of query qt0 it starts at)
   int ntiles;   // key tiles of 32 positions (0: no query of the sequence falls in this tile)
 };
-KVT_DEV QTile qtile_of(const void* cu_q, int cu_q_is_int64, const int32_t* kv_lens, int b, int qt, int qb) {
+KVT_DEV QTile qtile_of(const void* cu_q, int cu_q_is_int64, const int32_t* kv_lens, int b, int qt, int gs) {
   QTile Q;
   Q.qs = cu_q_is_int64 ? reinterpret_cast<const int64_t*>(cu_q)[b] : (int64_t)reinterpret_cast<const int32_t*>(cu_q)[b];
   const int64_t qe = cu_q_is_int64 ? reinterpret_cast<const int64_t*>(cu_q)[b + 1]
@@ -577,8 +582,20 @@ KVT_DEV QTile qtile_of(const void* cu_q, int cu_q_is_int64, const int32_t* kv_le
   Q.q_len = qe - Q.qs;
   Q.L = kv_lens[b];
   Q.q_pos0 = Q.L - Q.q_len;   // position of the chunk's first query
-  Q.qt0 = (int64_t)qt * qb;
-  Q.key_end = min(Q.L, Q.q_pos0 + min(Q.q_len, Q.qt0 + qb));   // keys visible to the tile's last query
+  // (unsigned 32-bit divisions: qt * 128 / gs = qt * (128 / gs) + qt * (128 % gs) / gs with qt < 2^27)
+  const uint32_t per = (uint32_t)kTileRows / (uint32_t)gs, left = (uint32_t)kTileRows % (uint32_t)gs;
+  int64_t qend;   // past the tile's last query
+  if (left == 0) {   // whole queries (gs divides 128): no division per tile
+    Q.qt0 = (int64_t)qt * per;
+    Q.rem = 0;
+    qend = Q.qt0 + per;
+  } else {
+    const uint32_t x = (uint32_t)qt * left;
+    Q.qt0 = (int64_t)qt * per + x / (uint32_t)gs;
+    Q.rem = (int)(x % (uint32_t)gs);
+    qend = Q.qt0 + ((uint32_t)Q.rem + kTileRows - 1) / (uint32_t)gs + 1;
+  }
+  Q.key_end = min(Q.L, Q.q_pos0 + min(Q.q_len, qend));   // keys visible to the tile's last query
   Q.ntiles = Q.qt0 < Q.q_len && Q.key_end > 0 ? (int)((Q.key_end + kT - 1) / kT) : 0;
   return Q;
 }
@@ -595,7 +612,6 @@ KVT_DEV void attend_segment(const KVSrc& S, const uint16_t* q, int64_t sq_n, int
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, kb = lane >> 4;
-  const int qpw = 16 / gs;   // queries per wavefront
   const int64_t qs = Q.qs, q_len = Q.q_len, L = Q.L, q_pos0 = Q.q_pos0, qt0 = Q.qt0, key_end = Q.key_end;
   constexpr uint32_t NG8 = kD / G8;
   bool pages_fit = true;   // the paged key range fits the kMaxLdsPages page ids staged in LDS
@@ -647,8 +663,8 @@ KVT_DEV void attend_segment(const KVSrc& S, const uint16_t* q, int64_t sq_n, int
   RawK rk_next = fetch_k<G8, BF16>(T, lds.pages, i0 * kT + tk, dc);
   RawV rv_next = fetch_v<G8, BF16>(T, lds.pages, i0 * kT + tp, db);
 
-  // ---- Q operands: row j of the wavefront's 16 = query qt0 + qpw wave + j / gs, head j % gs; channels
-  // 32 st + 8 kb .. + 7 of the row in one 16-byte load per st (the host checks the 16-byte alignment)
+  // ---- Q operands: row j of the wavefront's 16 = row t = rem + 16 wave + j counted from query qt0's first, i.e.
+  // query qt0 + t / gs, head t % gs; channels 32 st + 8 kb .. + 7 of the row in one 16-byte load per st (the host checks the 16-byte alignment)
   bf8 qop[8];
   int64_t qpos;   // position of this lane's query row (as the S^T column)
   // a paged range beyond the staged page ids would read clamped pages: the tile's outputs become NaN instead (NaN
@@ -657,9 +673,10 @@ KVT_DEV void attend_segment(const KVSrc& S, const uint16_t* q, int64_t sq_n, int
   {
     int gs_q = gs;                      // (computed per segment, not hoisted to the kernel start: see the output)
     asm volatile("" : "+s"(gs_q));
-    const int rq = n16 / gs_q, hq = n16 - rq * gs_q;
-    const int64_t qi = qt0 + (int64_t)qpw * wave + rq;
-    const bool ok = rq < qpw && qi < q_len;
+    const uint32_t t = (uint32_t)(Q.rem + 16 * wave + n16);
+    const int rq = (int)(t / (uint32_t)gs_q), hq = (int)t - rq * gs_q;
+    const int64_t qi = qt0 + rq;
+    const bool ok = qi < q_len;
     qpos = q_pos0 + qi;
     const uint16_t* qr = q + (qs + (ok ? qi : 0)) * sq_n + (int64_t)(h * gs + (ok ? hq : 0)) * sq_h + 8 * kb;
 #pragma unroll
@@ -957,7 +974,7 @@ KVT_DEV void attend_segment(const KVSrc& S, const uint16_t* q, int64_t sq_n, int
       for (int i = 0; i < 4; ++i) lrow[i] = Ls[i];
     }
   }
-  // ---- normalize and store: accumulator row r = 4 kb + i = query qt0 + qpw wave + r / gs, head r % gs;
+  // ---- normalize and store: accumulator row 4 kb + i of the wavefront's 16 (its query and head as for Q);
   // column n16 of block c = dim 16 c + n16
   // (one correctly rounded division per row: 128 / l, exact for a single visible key, where l = 1)
   // The rows' (query, head) split is computed here, after the key tiles: gs passes through an empty asm statement,
@@ -968,9 +985,10 @@ KVT_DEV void attend_segment(const KVSrc& S, const uint16_t* q, int64_t sq_n, int
   asm volatile("" : "+s"(gs_t), "+s"(out_t));
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int r = 4 * kb + i, rq = r / gs_t, hq = r - rq * gs_t;
-    const int64_t qi = qt0 + (int64_t)qpw * wave + rq;
-    if (rq < qpw && qi < q_len) {
+    const uint32_t t = (uint32_t)(Q.rem + 16 * wave + 4 * kb + i);
+    const int rq = (int)(t / (uint32_t)gs_t), hq = (int)t - rq * gs_t;
+    const int64_t qi = qt0 + rq;
+    if (qi < q_len) {
       const int64_t o0 = (qs + qi) * so_n + (int64_t)(h * gs_t + hq) * so_h;
       const float rl = 128.0f / lrow[i];
       if (out_f32) {
@@ -1007,7 +1025,6 @@ prefill_mfma_kernel(KVSrc S, const uint16_t* q, int64_t sq_n, int64_t sq_h, cons
   __shared__ int pfx[kMaxItems + 1];
   __shared__ int wsum[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int qb = kWaves * (16 / gs);
   const int n_items = bh_n * n_qtiles;
   int w = (int)blockIdx.x, G = 0, j;
   int64_t pos = 0, e = 0, T = 0;
@@ -1021,7 +1038,7 @@ prefill_mfma_kernel(KVSrc S, const uint16_t* q, int64_t sq_n, int64_t sq_h, cons
       cnt[k] = 0;
       if (k < per && jj < n_items) {
         const int bh = jj / n_qtiles, b = bh / H;
-        const int nt = qtile_of(cu_q, cu_q_is_int64, kv_lens, b, jj - bh * n_qtiles, qb).ntiles;
+        const int nt = qtile_of(cu_q, cu_q_is_int64, kv_lens, b, jj - bh * n_qtiles, gs).ntiles;
         cnt[k] = nt > 0 ? kItemCost + nt : 0;
       }
       sum += cnt[k];
@@ -1062,7 +1079,7 @@ prefill_mfma_kernel(KVSrc S, const uint16_t* q, int64_t sq_n, int64_t sq_h, cons
   }
   for (;;) {
     const int bh = j / n_qtiles, qt = j - bh * n_qtiles, b = bh / H, h = bh - b * H;
-    const QTile Q = qtile_of(cu_q, cu_q_is_int64, kv_lens, b, qt, qb);
+    const QTile Q = qtile_of(cu_q, cu_q_is_int64, kv_lens, b, qt, gs);
     int64_t p1 = Q.ntiles;
     int i0 = 0, nseg = 1, ord = 0;
     float* slots = nullptr;
@@ -1095,8 +1112,7 @@ prefill_mfma_kernel(KVSrc S, const uint16_t* q, int64_t sq_n, int64_t sq_h, cons
 // (kMaxItems), the same for every call, so the slots of one call never overlap the counters of another (a call with
 // more items than the previous one would otherwise find that call's slot data in its counters and merge early)
 int prefill_qtiles(int max_q, int H, int Hq) {
-  const int qb = kWaves * (16 / (Hq / H));   // queries per block
-  return (max_q + qb - 1) / qb;
+  return (int)(((int64_t)max_q * (Hq / H) + kTileRows - 1) / kTileRows);
 }
 constexpr int64_t kCounterBytes = (int64_t)kMaxItems * 4;   // 16 KB, a multiple of 256
 

@@ -116,6 +116,25 @@ def test_prefill_wide_groups(kvt_pkg, hq):
         assert torch.equal(outb, out.to(torch.bfloat16)), (hq, a)
 
 
+@pytest.mark.parametrize("hq", [2, 6, 10, 14, 22, 24, 30])
+@pytest.mark.parametrize("spread", [None, 0])
+def test_prefill_rows_across_queries(kvt_pkg, hq, spread):
+    """Query tiles are 128 (query, head) rows whatever query they start in: group sizes that do not divide 16 or 128
+    (1, 3, 5, 7, 11, 12, 15), chunks that end at and beside a tile's end, with and without a spread launch."""
+    from kvtier.kvt import kvt_prefill_attn
+    gs = hq // H
+    edge = 128 // gs
+    for a, n, xk, xv, dc, oc, gen in _chunked([edge, edge + 1, 2 * edge + 3, 1], 64, seed=18):
+        q = ref.make_q(hq, D, gen, n=n)
+        cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+        src = dict(k_src=xk.to(dev), v_src=xv.to(dev)) if a == 0 else {}
+        out = kvt_prefill_attn(dc, 0, q.to(dev), cu, out_dtype=torch.float32, spread=spread, **src).cpu()
+        kk, vv = (xk, xv) if a == 0 else oc.rows(0)
+        exp = _oracle_chunk(q, a, kk, vv)
+        err = (out - exp).abs()
+        assert float(err.max()) < 2e-3 and float(err.mean()) < 1e-3, (hq, a, float(err.max()), float(err.mean()))
+
+
 def test_prefill_first_query_closed_form(kvt_pkg):
     """Query 0 of a chunk without a prefix sees only key 0: the output is that V row (P = 1), for every q head of
     each KV head: exactly where |v| >= 2^-10 (v / 128 keeps its 8 significant bits in fp16), to 2^-18 below (fp16
