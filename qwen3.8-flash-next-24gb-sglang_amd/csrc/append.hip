@@ -7,8 +7,9 @@
 // division on the common path: scales from a * fl(1/qmax) and codes from x * rcp(s), each checked against the
 // rounding ties it could get wrong, with the IEEE division for the lanes that are close to one.
 //
-//   kvt_quant_store_tiered  dual write (patches/kv_tiers.py:272-443): owner stamp launch, then the INT8 ring row
-//                           (owner only) + INT4 pool row (always) launch.
+//   kvt_quant_store_tiered  dual write (patches/kv_tiers.py:272-443): the owner stamp (inside the write for up to
+//                           kScanTokens tokens, a launch before it for more), the INT8 ring row (owner only) and the
+//                           INT4 pool row (always).
 //   kvt_quant_store_int8    INT8-G quant + scatter (patches/kv_int8.py:281-362, with the fp16-max clamp).
 //   kvt_quant_store_int4    INT4-G32 quant + nibble pack + scatter (patches/kv_int4.py:289-393).
 //   kvt_page_table_update   writes (seq, logical page) -> physical page entries before an evicting append.
@@ -16,6 +17,8 @@
 //   kvt_append_evict        position-indexed ring append: requantizes the ring row being overwritten into the
 //                           INT4 page of its position (docs/KV_TIERS_PLAN.md:53, :63-67), then stores the new
 //                           token's INT8 row.
+
+#include <type_traits>
 
 #include "kvt_common.h"
 
@@ -275,13 +278,48 @@ __global__ void __launch_bounds__(256) stamp_owner_kernel(const void* loc, int l
   owner[slot & ring_mask] = (int32_t)slot;  // one winner per contested ring row (patches/kv_tiers.py:272-280)
 }
 
-// MODE 0: tiered dual write; 1: INT8 only (ring buffers are the pool); 2: INT4 only.  The row's slot index (and
-// in MODE 0 the owner word of its ring row) are wave-uniform scalar loads, issued behind the input loads; the
-// scheduling barriers keep the compiler from interleaving input-dependent arithmetic into that chain.
+// The owner stamp inside the dual write.  Every wavefront finds the winner of its own ring row among the N slots of
+// the call by itself: the last token whose slot falls in that ring row (any rule that all wavefronts share gives one
+// winner per row).  So nothing is read that another wavefront writes, and the stamp needs no launch of its own.  The
+// scan's loads go out together with the inputs'.  Returns the ring row's new owner word; *last: the winner's token.
+template <int LANES>
+KVT_DEV int32_t scan_owner(const void* loc, int loc64, uint32_t N, int64_t slot, int64_t ring_mask, int lane,
+                           uint32_t* last) {
+  constexpr int kAhead = 4;   // slots per lane in flight
+  uint32_t win = 0;
+  int32_t word = (int32_t)slot;   // (the row's own token matches, so some slot is always taken below)
+  for (uint32_t b = 0; b < N; b += kAhead * LANES) {
+    int64_t s[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) s[j] = load_loc(loc, loc64, min(b + (uint32_t)(j * LANES + lane), N - 1));
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t i = b + (uint32_t)(j * LANES + lane);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(i < N && ((s[j] ^ slot) & ring_mask) == 0);
+      if (m != 0) {
+        const int at = 63 - __builtin_clzll(m);
+        win = b + (uint32_t)(j * LANES + at);
+        word = __builtin_amdgcn_readlane((int32_t)s[j], at);
+      }
+    }
+  }
+  *last = win;
+  return word;
+}
+
+// Calls of at most this many tokens stamp inside the dual write, longer ones in a launch before it: the scan costs
+// every wavefront N slot reads, the launch 1.4 us whatever N (12 layers, two launches each against one: 56.7 -> 40.5 us
+// for 8 tokens, 62.0 -> 45.2 for 256, 68.1 -> 54.8 for 512, 78.9 -> 72.3 for 1,024, but 90.9 -> 111.6 for 2,048).
+constexpr int64_t kScanTokens = 1024;
+
+// MODE 0: tiered dual write after an owner stamp launch; 1: INT8 only (ring buffers are the pool); 2: INT4 only; 3:
+// tiered dual write with the stamp inside.  The row's slot index (and in MODE 0 the owner word of its ring row) are
+// wave-uniform scalar loads, issued behind the input loads; the scheduling barriers keep the compiler from
+// interleaving input-dependent arithmetic into that chain.
 template <int DT, int D, int G8, int MODE, int LM>
 __global__ void __launch_bounds__(256) quant_store_kernel(
     RowIn kin, RowIn vin, const void* loc, int loc64, uint32_t NH, int H, uint8_t* k4, uint8_t* v4, uint16_t* ks4,
-    uint16_t* vs4, int8_t* rk, int8_t* rv, uint16_t* rks, uint16_t* rvs, const int32_t* owner,
+    uint16_t* vs4, int8_t* rk, int8_t* rv, uint16_t* rks, uint16_t* rvs, int32_t* owner,
     const uint16_t* sm_k_inv, const uint16_t* sm_v_inv, int64_t ring_mask) {
   const int lane = threadIdx.x & 63;
   uint32_t t;
@@ -297,11 +335,17 @@ __global__ void __launch_bounds__(256) quant_store_kernel(
     __builtin_amdgcn_sched_barrier(0);
     hot = (int64_t)owner[slot & ring_mask] == slot;  // stamped by the preceding launch
   }
+  if constexpr (MODE == 3) {
+    uint32_t last;
+    const int32_t word = scan_owner<D / 4>(loc, loc64, NH / (uint32_t)H, slot, ring_mask, lane, &last);
+    hot = (int64_t)word == slot;
+    if (t == last && h == 0 && lane == 0) owner[slot & ring_mask] = word;
+  }
   __builtin_amdgcn_sched_barrier(0);
   float xk[4], xv[4];
   to_f32<DT, LM>(rk_in, xk);
   to_f32<DT, LM>(rv_in, xv);
-  if constexpr (MODE == 0) {
+  if constexpr (MODE == 0 || MODE == 3) {
     if (hot) {  // wave-uniform: the whole row belongs to one token
       store_ring_row<D, G8>(rk, rks, slot & ring_mask, H, h, lane, xk);
       store_ring_row<D, G8>(rv, rvs, slot & ring_mask, H, h, lane, xv);
@@ -490,7 +534,7 @@ int load_mode(const RowIn& kin, const RowIn& vin, int dtype, const void* smk, co
 template <int MODE>
 int launch_quant_store(const RowIn& kin, const RowIn& vin, int dtype, const void* loc, int loc64, int64_t N, int H,
                        int D, int group8, uint8_t* k4, uint8_t* v4, uint16_t* ks4, uint16_t* vs4, int8_t* rk,
-                       int8_t* rv, uint16_t* rks, uint16_t* rvs, const int32_t* owner, const uint16_t* smk,
+                       int8_t* rv, uint16_t* rks, uint16_t* rvs, int32_t* owner, const uint16_t* smk,
                        const uint16_t* smv, int64_t ring_mask, hipStream_t stream) {
   const dim3 grid((unsigned)((N * H + kWavesPerBlock - 1) / kWavesPerBlock));
   const int lm = load_mode(kin, vin, dtype, smk, smv);
@@ -553,15 +597,18 @@ int kvt_quant_store_tiered(const void* k, const void* v, int dtype, int64_t sk_n
   if (N < 0 || H <= 0 || N > INT32_MAX / H || ring_mask < 0 || ((ring_mask + 1) & ring_mask) != 0) return KVT_EINVAL;
   if (N == 0) return KVT_OK;
   hipStream_t st = (hipStream_t)stream;
+  const auto store = [&](auto mode) {
+    return launch_quant_store<decltype(mode)::value>(
+        RowIn{k, sk_n, sk_h}, RowIn{v, sv_n, sv_h}, dtype, loc, loc_is_int64, N, H, D, group8, (uint8_t*)k_buf,
+        (uint8_t*)v_buf, (uint16_t*)k_scale, (uint16_t*)v_scale, (int8_t*)ring_k, (int8_t*)ring_v, (uint16_t*)ring_ks,
+        (uint16_t*)ring_vs, (int32_t*)owner, (const uint16_t*)sm_k_inv, (const uint16_t*)sm_v_inv, ring_mask, st);
+  };
+  if (N <= kScanTokens) return store(std::integral_constant<int, 3>{});
   const unsigned sblocks = (unsigned)((N + 255) / 256);
   hipLaunchKernelGGL(stamp_owner_kernel, dim3(sblocks), dim3(256), 0, st, loc, loc_is_int64, N, (int32_t*)owner,
                      ring_mask);
   KVT_CHECK_LAUNCH();
-  return launch_quant_store<0>(RowIn{k, sk_n, sk_h}, RowIn{v, sv_n, sv_h}, dtype, loc, loc_is_int64, N, H, D, group8,
-                               (uint8_t*)k_buf, (uint8_t*)v_buf, (uint16_t*)k_scale, (uint16_t*)v_scale,
-                               (int8_t*)ring_k, (int8_t*)ring_v, (uint16_t*)ring_ks, (uint16_t*)ring_vs,
-                               (const int32_t*)owner, (const uint16_t*)sm_k_inv, (const uint16_t*)sm_v_inv,
-                               ring_mask, st);
+  return store(std::integral_constant<int, 0>{});
 }
 
 int kvt_quant_store_int8(const void* k, const void* v, int dtype, int64_t sk_n, int64_t sk_h, int64_t sv_n,

@@ -165,6 +165,44 @@ def test_tiered_boundary_and_collisions(kvt_pkg):
     assert contested > 100
 
 
+@pytest.mark.parametrize("n,loc_dtype,dt,g8", [(1, torch.int32, torch.bfloat16, 64), (63, torch.int64, torch.bfloat16, 64),
+                                               (257, torch.int32, torch.float16, 256), (256, torch.int32, torch.float32, 64),
+                                               (1024, torch.int64, torch.bfloat16, 64), (1025, torch.int32, torch.bfloat16, 64)])
+def test_tiered_stamp_inside_the_write(kvt_pkg, n, loc_dtype, dt, g8):
+    """Writes of up to 1,024 tokens stamp the owner inside the dual write, longer ones in a launch before it: sizes at
+    the scan's group edges and on both sides of that line, half of the ring rows contested.  One winner per ring row
+    among its writers, its row bit-exact in both tensors, rows nobody wrote untouched, every INT4 row exact."""
+    from kvtier import sparse_attn as sa
+    gen = torch.Generator().manual_seed(70 + n)
+    R, slots = 2048, 16384
+    k = (torch.randn(n, H, D, generator=gen) * 3).to(dt)
+    v = (torch.randn(n, H, D, generator=gen) * 3).to(dt)
+    ones = torch.ones(H, D, dtype=torch.float16, device=dev)
+    i = torch.randperm(n, generator=gen)                       # tokens 2 j and 2 j + 1 (in some order) share ring row j
+    member = torch.randint(0, slots // R, (n,), generator=gen)[i // 2] + i % 2
+    loc = member % (slots // R) * R + i // 2
+    b = _bufs(slots, R, g8)
+    sa.quant_store_kv_tiered(k.to(dev), v.to(dev), loc.to(loc_dtype).to(dev), *b, ones, ones, R - 1)
+    torch.cuda.synchronize()
+    c = _cpu(b)
+    for t, x in enumerate((k, v)):
+        p4, s4 = ref.quant4(x)
+        assert torch.equal(c[t][loc], p4) and torch.equal(c[2 + t][loc], s4)
+    owner = c[8].long()
+    written = torch.zeros(R, dtype=torch.bool)
+    written[loc % R] = True
+    assert torch.equal(owner >= 0, written)
+    at = torch.full((slots,), -1, dtype=torch.long)
+    at[loc] = torch.arange(n)
+    own = owner[written]
+    assert torch.equal(own % R, torch.nonzero(written).flatten()) and (at[own] >= 0).all()
+    for t, x in enumerate((k, v)):
+        q8, s8 = ref.quant8(x, group=g8)
+        assert torch.equal(c[4 + t][own % R], q8[at[own]]) and torch.equal(c[6 + t][own % R], s8[at[own]])
+        fill, scale = ((0x33, 7.0), (0x44, 9.0))[t]
+        assert (c[4 + t][~written] == fill).all() and (c[6 + t][~written] == scale).all()
+
+
 def test_fp16_max_clamp_writers(kvt_pkg):
     """1e6 / bf16-max groups: ring and INT4 scales 65504, codes bit-exact vs the clamped references
     (gemv/test_kv_tiers.py:412-436)."""
