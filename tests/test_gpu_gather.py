@@ -191,6 +191,30 @@ def test_prefix_gather_tiered_gaps(tiered_state):
     assert torch.isnan(pk[~written]).all() and torch.isnan(pv[~written]).all()
 
 
+def test_gathers_unaligned_smoothing(tiered_state):
+    """Smoothing factors at an odd element offset (2-byte aligned only) give the rows of aligned ones, bit for bit."""
+    from kvtier import sparse_attn as sa
+    st = tiered_state
+    lens = torch.tensor([37, 200], dtype=torch.int32, device=dev)
+    r2t = torch.randint(0, SLOTS, (2, 200), dtype=torch.int32, generator=st["gen"]).to(dev)
+    req = torch.arange(2, device=dev)
+    cu = torch.tensor([0, 37, 237], dtype=torch.int32, device=dev)
+    outs = []
+    for shift in (0, 1):
+        buf = [torch.zeros(H * D + 1, dtype=torch.float16, device=dev) for _ in range(2)]
+        sm = [t[shift:shift + H * D].view(H, D) for t in buf]
+        sm[0].copy_(st["sm_k"]), sm[1].copy_(st["sm_v"])
+        out = [torch.zeros(237, H, D, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        sa.qwen_sparse_prefix_gather_dequant_tiered(
+            st["k4"], st["v4"], st["ks4"], st["vs4"], *sm, r2t, req, lens, cu, *out, 2, 200, ring_k=st["rk"],
+            ring_v=st["rv"], ring_ks=st["rks"], ring_vs=st["rvs"], owner=st["owner"], ring_mask=R - 1)
+        outs.append([t.cpu().view(torch.int16) for t in out])
+    slots = torch.cat([r2t[0, :37], r2t[1]]).cpu().long()
+    assert torch.equal(outs[0][0], st["dk_all"][slots].view(torch.int16))
+    assert torch.equal(outs[0][1], st["dv_all"][slots].view(torch.int16))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 def test_single_tier_gathers(tiered_state):
     """int4 and int8 pool gathers (compact + prefix) bit-exact vs the oracle's dequant (gemv/test_kv_int4.py:140-247,
     gemv/test_kv_int8.py:101-163)."""
