@@ -242,9 +242,12 @@ bool aligned_args(int kind, const void* k, const void* v, const void* rk, const 
 
 
 // counts[b] = #{c < topk : 0 <= indices[b * idx_stride + c] < seq_lens[b]}; cu_k[0] = 0, cu_k[b + 1] = counts[0] + ..
-// + counts[b].  One block of kCuThreads: rows go to the wavefronts in turn (64 columns per coalesced load, a wavefront
-// sum per row), then the block scans a chunk of kCuThreads counts in LDS (Hillis-Steele, double-buffered) and adds
-// the running total of the earlier chunks.
+// + counts[b].  One block of kCuThreads, kCuThreads rows at a time: a row's columns go to one wavefront, or to several
+// where there are more wavefronts than rows, in chunks of 64 kCuAhead columns whose loads are in flight together (the
+// launch is a few dependent memory rounds long: 8 rows of 2,051 columns took 13.7 us with one load per round and one
+// wavefront per row, 7.0 us now); then the block scans the chunk's counts in LDS (Hillis-Steele, double-buffered)
+// and adds the running total of the earlier chunks.
+constexpr int kCuAhead = 16;
 constexpr int kCuThreads = 1024;
 
 __global__ void __launch_bounds__(kCuThreads) cu_seqlens_kernel(const int32_t* seq_lens, const int32_t* indices,
@@ -261,30 +264,32 @@ __global__ void __launch_bounds__(kCuThreads) cu_seqlens_kernel(const int32_t* s
   int64_t carry = 0;
   for (int r0 = 0; r0 < batch; r0 += kCuThreads) {
     const int nrows = min(kCuThreads, batch - r0);
-    for (int r = wave; r < nrows; r += kW) {
-      const int b = r0 + r;
+    buf[0][t] = 0;
+    __syncthreads();
+    const int split = nrows < kW ? kW / nrows : 1;   // wavefronts per row
+    for (int item = wave; item < nrows * split; item += kW) {
+      const int r = item / split, b = r0 + r;
       const int64_t L = seq_lens[b];
       const int32_t* row = indices + (int64_t)b * idx_stride;
       int n = 0;
-      for (int c0 = 0; c0 < topk; c0 += 64) {
-        const int c = c0 + lane;
-        if (c < topk) {
-          const int64_t p = row[c];
-          n += (p >= 0 && p < L) ? 1 : 0;
+      for (int64_t c0 = (int64_t)(item - r * split) * 64 * kCuAhead; c0 < topk; c0 += (int64_t)split * 64 * kCuAhead) {
+        int32_t p[kCuAhead];
+#pragma unroll
+        for (int j = 0; j < kCuAhead; ++j) {   // (past the end: the last column, not counted)
+          const int64_t c = c0 + 64 * j + lane;
+          p[j] = row[c < topk ? c : topk - 1];
         }
+#pragma unroll
+        for (int j = 0; j < kCuAhead; ++j) n += (c0 + 64 * j + lane < topk && p[j] >= 0 && (int64_t)p[j] < L) ? 1 : 0;
       }
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-      if (lane == 0) {
-        buf[0][r] = n;
-        counts[b] = n;
-      }
+      if (lane == 0) atomicAdd(&buf[0][r], n);
     }
     __syncthreads();
     int cur = 0;
-    if (t >= nrows) buf[0][t] = 0;
-    __syncthreads();
-    for (int d = 1; d < kCuThreads; d <<= 1) {
+    if (t < nrows) counts[r0 + t] = buf[0][t];
+    for (int d = 1; d < nrows; d <<= 1) {   // (entries past nrows are zero)
       const int v = buf[cur][t] + (t >= d ? buf[cur][t - d] : 0);
       buf[cur ^ 1][t] = v;
       cur ^= 1;
