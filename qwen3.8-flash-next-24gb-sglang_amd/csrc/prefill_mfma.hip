@@ -1127,7 +1127,10 @@ int kvt_prefill_work_bytes(int batch, int H, int Hq, int max_q, int spread_block
     *bytes = 0;
     return KVT_OK;
   }
-  const int64_t n_items = (int64_t)batch * H * prefill_qtiles(max_q, H, Hq);
+  // sized for tiles of whole queries (8 wavefronts x 16 / gs queries, at least as many tiles as of 128 rows each), the
+  // size and the item limit that callers have always been given
+  const int qb = kWaves * (16 / (Hq / H));
+  const int64_t n_items = (int64_t)batch * H * (((int64_t)max_q + qb - 1) / qb);
   if (n_items > kMaxItems || spread_blocks > (1 << 20)) return KVT_ERANGE;
   *bytes = kCounterBytes + (n_items + spread_blocks - 1) * kSlotFloats * 4;
   return KVT_OK;

@@ -779,7 +779,7 @@ def kvt_prefill_attn(cache: PosTieredCache, layer: int, q: torch.Tensor, cu_q: t
     if batch == 0 or max_q == 0:
         return out
     if spread is None:
-        spread = prefill_spread_blocks(-(-int(max_q) * (Hq // H) // 128) * batch * H, q.device)
+        spread = prefill_spread_blocks(-(-max_q // (8 * (16 // (Hq // H)))) * batch * H, q.device)
     need = ctypes.c_int64(0)
     _lib.call("kvt_prefill_work_bytes", batch, H, Hq, int(max_q), int(spread), ctypes.byref(need))
     if need.value and work is None:
