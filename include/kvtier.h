@@ -135,7 +135,8 @@ int kvt_compact_gather(int kind, const void* k, const void* v, const void* k_sca
  * out_bf16 (exactly one; [batch, Hq, D] rows with batch stride out_stride_b >= Hq * D, a multiple of 8, 16-byte
  * aligned); calls sharing the counters and
  * partials must not overlap.  Faster than the combine launch for few splits (<= 8), slower for many: one block
- * reads all of a (request, KV head)'s partials.  A request with no attended column comes out
+ * reads all of a (request, KV head)'s partials.  cu_k NULL: every column counts (column c of request b is attended
+ * when 0 <= indices[b][c] < seq_lens[b]).  A request with no attended column comes out
  * NaN (0/0).  n_splits >= 1; Hq / H <= 16, D = 256.  Kinds and buffers as kvt_compact_gather; pool_rows = rows of k / v (byte offsets
  * are 32-bit: pool_rows * H * D (INT8) or * D / 2 (INT4) < 2^31, else KVT_ERANGE).  No reference counterpart: it replaces the
  * compact gather + FlashAttention-2 pair of the reference's decode (flat patch
@@ -296,7 +297,8 @@ int kvt_prefill_attn(const void* q, int64_t sq_n, int64_t sq_h, const void* cu_q
 
 /* Bytes of the kvt_prefill_attn workspace for these shapes and spread_blocks (0 for spread_blocks 0): a zeroed
  * 4-byte counter per (sequence, KV head, query tile of 128 rows), padded to 256 bytes, and a 132,096-byte state
- * slot (O, m, l of 128 rows in fp32) per query tile plus one per block beyond the first.  No counterpart in the
+ * slot (O, m, l of 128 rows in fp32) per query tile plus one per block beyond the first, query tiles counted as of
+ * 8 * (16 / (Hq / H)) whole queries (at least as many as the launch has).  No counterpart in the
  * reference (its prefill kernel takes one block per query row). */
 int kvt_prefill_work_bytes(int batch, int H, int Hq, int max_q, int spread_blocks, int64_t* bytes);
 

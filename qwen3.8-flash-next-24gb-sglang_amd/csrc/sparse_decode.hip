@@ -75,8 +75,9 @@ struct SparseArgs {
   const int32_t* indices;  // [batch, idx_stride], the first topk columns used
   int64_t idx_stride;
   const int32_t* seq_lens;
-  const void* cu_k;
-  int cu64;
+  const void* cu_k;        // decode: the valid counts' prefix sum; null at the entry point: every column counts (the
+  int cu64;                // launcher then points it at seq_lens, whose entry b is read for both bounds and not used)
+  int all_columns;
   int topk;
   int H;
   int gs;
@@ -661,7 +662,7 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
   // the first tile's resolve chain (position, slot, owner).  The q rows reach LDS after the chain.
   const IdxWords wreq = idx_words(A.req_indices, A.req64, b);
   const IdxWords w0 = ROWS ? idx_words(A.cu_q, A.cuq64, b) : idx_words(A.cu_k, A.cu64, b);
-  const IdxWords w1 = ROWS ? idx_words(A.cu_q, A.cuq64, b + 1) : idx_words(A.cu_k, A.cu64, b + 1);
+  const IdxWords w1 = ROWS ? idx_words(A.cu_q, A.cuq64, b + 1) : idx_words(A.cu_k, A.cu64, b + 1 - A.all_columns);
   const int32_t len = ROWS ? A.kv_lens[b] : A.seq_lens[b];   // widened after the barrier (no wait before it)
   // the group's q heads (512 16-byte chunks, 2 per thread; heads beyond the group read head 0 and are zeroed)
   constexpr int kQChunks = kHeads * kD / 8 / (64 * kWaves);
@@ -695,7 +696,7 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     c_end = visible < (int64_t)A.topk ? (visible > 0 ? visible : 0) : (int64_t)A.topk;
   } else {
     qrow = b;
-    const int64_t vcount = x1 - x0;
+    const int64_t vcount = A.all_columns != 0 ? L : x1 - x0;
     const int64_t span = (int64_t)kCols * (MULTI ? A.tiles : 1);
     c_begin = (int64_t)wx * span;
     const int64_t lim = vcount < (int64_t)A.topk ? vcount : (int64_t)A.topk;
@@ -982,7 +983,8 @@ int kvt_sparse_decode(int kind, const void* q, int64_t q_stride_b, const void* k
   A.sm_k = (const uint16_t*)sm_k, A.sm_v = (const uint16_t*)sm_v;
   A.req_to_token = (const int32_t*)req_to_token, A.req_stride = req_stride, A.req_indices = req_indices;
   A.req64 = req_is_int64 != 0, A.indices = (const int32_t*)indices, A.idx_stride = idx_stride;
-  A.seq_lens = (const int32_t*)seq_lens, A.cu_k = cu_k, A.cu64 = cu_is_int64 != 0, A.topk = topk;
+  A.seq_lens = (const int32_t*)seq_lens, A.cu_k = cu_k != nullptr ? cu_k : seq_lens, A.cu64 = cu_k != nullptr && cu_is_int64 != 0;
+  A.all_columns = cu_k == nullptr, A.topk = topk;
   A.H = H, A.gs = Hq / H, A.n_splits = n_splits, A.tiles = tiles, A.rows8 = (uint32_t)rows8;
   A.rows4 = (uint32_t)rows4, A.scale = scale, A.q = (const uint16_t*)q, A.sq_n = q_stride_b, A.sq_h = kD;
   A.si_m = idx_stride, A.si_g = 0, A.si_n = 1, A.part_o = (float*)part_o, A.part_ml = (float*)part_ml;

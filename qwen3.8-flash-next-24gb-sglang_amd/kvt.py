@@ -665,20 +665,15 @@ def decode_attn_slots(q, seq_lens, req_to_token, req_indices, k4, v4, ks4, vs4, 
             raise ValueError("decode_attn_slots: pass max_len (a host int >= every seq_len) under graph capture")
         max_len = int(seq_lens.max())   # one device reduction and synchronization
     if impl == "mfma":
-        from .sparse_attn import qwen_sparse_decode_attn
+        from .sparse_attn import ALL_COLUMNS, qwen_sparse_decode_attn
         ws = workspace if workspace is not None else {}
         idx = ws.get("dense_idx")
         if idx is None or idx.shape[1] < max_len or idx.device != q.device:
             idx = torch.arange(max_len, dtype=torch.int32, device=q.device)[None]
             ws["dense_idx"] = idx
-        cu = ws.get("dense_cu")
-        if cu is None or cu.numel() != B + 1 or cu.device != q.device:
-            cu = torch.zeros(B + 1, dtype=torch.int32, device=q.device)
-            ws["dense_cu"] = cu
-        torch.cumsum(seq_lens.clamp(max=max_len), 0, dtype=torch.int32, out=cu[1:])
         out = torch.empty(B, Hq, D, dtype=out_dtype, device=q.device)
         return qwen_sparse_decode_attn(q, k4, v4, req_to_token, req_indices, idx[:, :max_len].expand(B, max_len),
-                                       seq_lens, cu, B, max_len, k_scale=ks4, v_scale=vs4, sm_k=sm_k, sm_v=sm_v,
+                                       seq_lens, ALL_COLUMNS, B, max_len, k_scale=ks4, v_scale=vs4, sm_k=sm_k, sm_v=sm_v,
                                        kv_bits=4, ring_k=rk, ring_v=rv, ring_ks=rks, ring_vs=rvs, owner=owner,
                                        ring_mask=ring_mask, out=out, workspace=ws)
     if impl != "ref":

@@ -216,6 +216,7 @@ def qwen_sparse_kv_extraction_compact_triton(
               out_v.data_ptr(), _lib.stream())
 
 
+ALL_COLUMNS = object()   # as cu_k of qwen_sparse_decode_attn: column c counts whenever indices[b, c] < seq_lens[b]
 _MULTI_BLOCKS = 512   # blocks of a long-selection launch: one per resident slot, 2 per CU (256 VGPRs)
 
 
@@ -235,7 +236,7 @@ def qwen_sparse_decode_attn(
     combine launch, whose blocks (one per request, q head and slice of dims) read the partials side by side.
 
     q: bf16 [batch, Hq, D]; the pool/ring/owner/scale arguments as the compact gather; cu_k: the valid counts'
-    prefix sum (qwen_sparse_fa2_cu_seqlens_triton).  Column c of request b is attended when c < cu_k[b+1] - cu_k[b]
+    prefix sum (qwen_sparse_fa2_cu_seqlens_triton), or ALL_COLUMNS.  Column c of request b is attended when c < cu_k[b+1] - cu_k[b]
     and 0 <= indices[b, c] < seq_lens[b].  Returns out (fp32 [batch, Hq, D] unless a bf16/fp32 `out` is given);
     a request with no attended column gives NaN.  `workspace` (a dict) keeps the partial buffers across calls;
     `splits` sets the number of column splits per (request, KV head) instead of the launch-size rule below."""
@@ -298,7 +299,7 @@ def qwen_sparse_decode_attn(
         if ws.get("sparse_ctr") is None or ws["sparse_ctr"].numel() < batch * heads:
             ws["sparse_ctr"] = torch.zeros(batch * heads, dtype=torch.int32, device=q.device)   # each call leaves 0
     rq, rq64 = _idx_args(req_indices)
-    cu, cu64 = _idx_args(cu_k)
+    cu, cu64 = (None, 0) if cu_k is ALL_COLUMNS else _idx_args(cu_k)
     tier = kind == _KIND_TIERED
     smk = None if sm_k is None else sm_k.contiguous()
     smv = None if sm_v is None else sm_v.contiguous()

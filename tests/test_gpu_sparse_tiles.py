@@ -65,3 +65,26 @@ def test_tile_edges(kvt_pkg, kind, tiers, identity):
             a["v_scale"], a["sm_k"], a["sm_v"], a["kv_bits"], **{k: a[k] for k in a if k.startswith(("ring_", "owner"))},
             splits=splits, out=torch.empty(n, HQ, D, device=dev))
         close(got.cpu(), exp)
+
+
+def test_all_columns_equals_counted(kvt_pkg):
+    """ALL_COLUMNS in place of the valid counts (every position selected) gives the counted call's output bit for bit:
+    lengths 0 (NaN), 1, at and beside a tile's end, and beyond the selection's width."""
+    from kvtier import sparse_attn as sa
+    gen = torch.Generator().manual_seed(72)
+    R, slots, width = 1024, 4096, 700
+    p = slot_pools(slots, R, 64, gen)
+    lens = torch.tensor([0, 1, 16, 17, 640, 699, 700, 900], dtype=torch.int32)
+    n = lens.numel()
+    r2t = torch.stack([torch.randperm(slots, generator=gen)[:1000] for _ in range(n)]).to(torch.int32).to(dev)
+    idx = torch.arange(width, dtype=torch.int32, device=dev)[None].expand(n, width)
+    cu = torch.nn.functional.pad(lens.clamp(max=width).cumsum(0), (1, 0)).to(torch.int32).to(dev)
+    q = (torch.randn(n, HQ, D, generator=gen) / 4).to(torch.bfloat16).to(dev)
+    a = pool_args("tiered", p, R, dev)
+    ring = {k: a[k] for k in a if k.startswith(("ring_", "owner"))}
+    for splits in (None, 2):   # one tile per wavefront; several
+        out = [sa.qwen_sparse_decode_attn(q, a["k_buf"], a["v_buf"], r2t, torch.arange(n, device=dev), idx, lens.to(dev), c,
+                                          n, width, a["k_scale"], a["v_scale"], a["sm_k"], a["sm_v"], 4, splits=splits,
+                                          **ring).cpu() for c in (cu, sa.ALL_COLUMNS)]
+        assert torch.isnan(out[0][0]).all() and not torch.isnan(out[0][1:]).any()
+        assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
