@@ -18,9 +18,8 @@ KVT_DEV uint32_t bf16x2(float lo, float hi) {
 // into the mantissa of an fp16 magic value h = 1024 + (c + o) (v_perm_b32 for bytes, v_and_or_b32 for nibbles), in
 // pairs of channels (0, 2), (1, 3), (4, 6), (5, 7); v_fma_mix_f32 converts h and s and computes
 // h * s - (1024 + o) * s in one rounding, whose exact value c * s is representable (4 or 8 bits times the scale's
-// 11), so the fp32 product equals the plain c * s; the smoothing factor then multiplies in fp32 (SM; a product with 1
-// changes nothing, so identity factors take the body without it) and v_cvt_pk_bf16_f32 rounds each pair to nearest
-// even.
+// 11), so the fp32 product equals the plain c * s; the caller then multiplies by the smoothing factor in fp32 and
+// rounds each pair to nearest even with v_cvt_pk_bf16_f32.
 KVT_DEV uint32_t and_or(uint32_t x, uint32_t m, uint32_t o) {
   uint32_t r;
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(m), "v"(o));
@@ -37,7 +36,7 @@ KVT_DEV void magic8(uint2 w, uint32_t m[4]) {
   m[2] = __builtin_amdgcn_perm(0x64646464u, v, 0x04020400u);
   m[3] = __builtin_amdgcn_perm(0x64646464u, v, 0x04030401u);
 }
-KVT_DEV void magic4(uint32_t w, uint32_t m[4]) {   // pairs (0, 4), (1, 5), (2, 6), (3, 7): one instruction less
+KVT_DEV void magic4(uint32_t w, uint32_t m[4]) {   // pairs (0, 4), (1, 5), (2, 6), (3, 7), one instruction less than magic8's
   m[0] = and_or(w, 0x000F000Fu, 0x64006400u);
   m[1] = and_or(w >> 4, 0x000F000Fu, 0x64006400u);
   m[2] = and_or(w >> 8, 0x000F000Fu, 0x64006400u);
