@@ -137,7 +137,8 @@ KVT_DEV void magic4_as8(uint32_t w, uint32_t m[4]) {   // in magic8's pairs
   m[3] = and_or(b >> 4, 0x000F000Fu, 0x64006400u);
 }
 // The 8 channels of magic words m (PAIRS4: magic4's pairs, else magic8's) as bf16; SM: times the smoothing factors (a
-// product with 1 changes nothing, so identity factors take the body without it).  offset: 1024 + o (exact products, as the scale's 11 bits times 1032 or 1152 = 9 * 128 fit fp32)
+// product with 1 changes nothing, so identity factors take the body without it).  offset: 1024 + o (exact products: the
+// scale's 11 bits times 1032 or 1152 fit fp32).
 template <bool SM, bool PAIRS4>
 KVT_DEV uint4 rows_bf16(const uint32_t m[4], uint32_t sbits, float offset, const uint4& sm) {
   const _Float16 s = __builtin_bit_cast(_Float16, (uint16_t)(sbits & 0xffffu));
