@@ -17,7 +17,7 @@
 //   kvt_sparse_cu_seqlens  valid top-k counts and their prefix sum, the offsets kvt_compact_gather packs at (the
 //                       upstream qwen_sparse_fa2_cu_seqlens_triton the reference calls first, gemv/test_kv_tiers.py:297-301)
 
-#include "dequant_common.h"
+#include "kvt_common.h"
 
 using namespace kvt;
 
@@ -75,27 +75,22 @@ KVT_DEV Raw load_int4(const uint8_t* codes, const uint16_t* scales, int64_t row,
   return r;
 }
 
-// q * s * sm in fp32 (patches/kv_tiers.py:519-525), the product q * s exact
-KVT_DEV uint4 dequant8(const Raw& r, const float m[8]) {
-  uint32_t w[4];
-  magic8(r.w, w);
-  const _Float16 s = __builtin_bit_cast(_Float16, r.s);
-  const float c = fmaf((float)s, -1152.0f, 0.0f);
-  return make_uint4(bf16x2(mix(w[0], 0, s, c) * m[0], mix(w[1], 0, s, c) * m[1]),
-                    bf16x2(mix(w[0], 1, s, c) * m[2], mix(w[1], 1, s, c) * m[3]),
-                    bf16x2(mix(w[2], 0, s, c) * m[4], mix(w[3], 0, s, c) * m[5]),
-                    bf16x2(mix(w[2], 1, s, c) * m[6], mix(w[3], 1, s, c) * m[7]));
+// The product of code and scale is formed as such: folding the codes' offset into one fma (h s - 1152 s) is as exact for
+// finite scales, but gives NaN for every code of an infinite one and +0 for a negative code of a zero one.
+KVT_DEV uint4 dequant8(const Raw& r, const float m[8]) {   // q * s * sm (patches/kv_tiers.py:525)
+  const float s = f16_bits_to_f32(r.s);
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = (float)(int8_t)((i < 4 ? r.w.x : r.w.y) >> (8 * (i & 3))) * s * m[i];
+  return make_uint4(bf16x2(x[0], x[1]), bf16x2(x[2], x[3]), bf16x2(x[4], x[5]), bf16x2(x[6], x[7]));
 }
 
-KVT_DEV uint4 dequant4(const Raw& r, const float m[8]) {
-  uint32_t w[4];
-  magic4(r.w.x, w);
-  const _Float16 s = __builtin_bit_cast(_Float16, r.s);
-  const float c = fmaf((float)s, -1032.0f, 0.0f);
-  return make_uint4(bf16x2(mix(w[0], 0, s, c) * m[0], mix(w[1], 0, s, c) * m[1]),
-                    bf16x2(mix(w[2], 0, s, c) * m[2], mix(w[3], 0, s, c) * m[3]),
-                    bf16x2(mix(w[0], 1, s, c) * m[4], mix(w[1], 1, s, c) * m[5]),
-                    bf16x2(mix(w[2], 1, s, c) * m[6], mix(w[3], 1, s, c) * m[7]));
+KVT_DEV uint4 dequant4(const Raw& r, const float m[8]) {   // ((b & 15) - 8) * s * sm (patches/kv_tiers.py:519-523)
+  const float s = f16_bits_to_f32(r.s);
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = (float)((int)((r.w.x >> (4 * i)) & 15u) - 8) * s * m[i];
+  return make_uint4(bf16x2(x[0], x[1]), bf16x2(x[2], x[3]), bf16x2(x[4], x[5]), bf16x2(x[6], x[7]));
 }
 
 // 8 smoothing factors as fp32: one 16-byte load where the tensor is 16-byte aligned (sm16), else element loads (the

@@ -93,6 +93,13 @@ KVT_DEV uint32_t pack_pair(float qe, float qo) {
   return (uint32_t)((int)qe + 8) | ((uint32_t)((int)qo + 8) << 4);
 }
 
+// bf16 pair (round to nearest even, one v_cvt_pk_bf16_f32): lo in bits 0-15.
+KVT_DEV uint32_t bf16x2(float lo, float hi) {
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){lo, hi}, bf2v));
+}
+
 }  // namespace kvt
 
 // Status codes returned by every C-ABI entry point (mapped to Python exceptions by the wrappers).

@@ -8,6 +8,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from kvt_testutil import pool_args, slot_pools, slot_rows
 from oracle import ref
 
 pytestmark = pytest.mark.gpu
@@ -213,6 +214,38 @@ def test_gathers_unaligned_smoothing(tiered_state):
     assert torch.equal(outs[0][0], st["dk_all"][slots].view(torch.int16))
     assert torch.equal(outs[0][1], st["dv_all"][slots].view(torch.int16))
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("kind", ["tiered", "int4", "int8"])
+def test_gathers_extreme_scales(kvt_pkg, kind):
+    """Rows whose fp16 scales are infinite, NaN, zero, subnormal or the largest finite value, with every code: bf16(code
+    * scale * smoothing) exactly as the oracle forms it (an infinite scale: signed infinities and NaN for code 0; a zero
+    scale: zeros of the code's sign), NaN for NaN and every other entry bit for bit, by both gathers."""
+    from kvtier import sparse_attn as sa
+    gen = torch.Generator().manual_seed(73)
+    rings, slots = 64, 256
+    p = slot_pools(slots, rings, 64, gen)
+    scales = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, 2.0 ** -24, 65504.0, 1.0])
+    for name in ("ks4", "vs4", "rks", "rvs", "ks8", "vs8"):
+        p[name] = scales[torch.randint(0, len(scales), p[name].shape, generator=gen)].half()
+    r2t = torch.randperm(slots, generator=gen)[None].to(torch.int32)
+    exp = slot_rows(kind, p, r2t[0], rings, 64)
+    a = pool_args(kind, p, rings, dev)
+    ring = {k: a[k] for k in a if k.startswith(("ring_", "owner"))}
+    out = [torch.zeros(slots, H, D, dtype=torch.bfloat16, device=dev) for _ in range(4)]
+    req, lens = torch.zeros(1, dtype=torch.int64, device=dev), torch.tensor([slots], dtype=torch.int32, device=dev)
+    cu = torch.tensor([0, slots], dtype=torch.int32, device=dev)
+    getattr(sa, "qwen_sparse_prefix_gather_dequant_" + kind)(
+        a["k_buf"], a["v_buf"], a["k_scale"], a["v_scale"], a["sm_k"], a["sm_v"], r2t.to(dev), req, lens, cu, *out[:2],
+        1, slots, **ring)
+    idx = torch.arange(slots, dtype=torch.int32, device=dev)[None]
+    sa.qwen_sparse_kv_extraction_compact_triton(
+        a["k_buf"], a["v_buf"], r2t.to(dev), req, idx, lens, cu, *out[2:], 1, slots, a["k_scale"], a["v_scale"],
+        a["sm_k"], a["sm_v"], a["kv_bits"], **ring)
+    for got, want in zip((t.cpu() for t in out), exp * 2):
+        nan = torch.isnan(want)
+        assert torch.equal(nan, torch.isnan(got)) and nan.any() and torch.isinf(want).any()
+        assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
 
 
 def test_single_tier_gathers(tiered_state):
