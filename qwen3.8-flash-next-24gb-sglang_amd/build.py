@@ -6,6 +6,7 @@ Every .hip file under csrc/ is compiled to an object with hipcc (in parallel), t
   -fhip-fp32-correctly-rounded-divide-sqrt    IEEE fp32 division (the quantizers' x / s must be exact)
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                               no packed fp32 VALU instructions
+  -Werror=unused-function                     a helper that nothing calls fails the build
   no -ffast-math: rounding must follow IEEE round-to-nearest-even.
 Per file: decode_mfma.hip, decode_rows.hip and decode_ref.hip preload the first kernel-argument dwords into SGPRs
 (-mllvm -amdgpu-kernarg-preload-count=16; the split-K kernel's arguments are ordered for it).
@@ -34,7 +35,7 @@ CFLAGS = [
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall",
-    "-Wno-unused-function",
+    "-Werror=unused-function",
     f"-I{CSRC}",
     f"-I{INCLUDE}",
 ]

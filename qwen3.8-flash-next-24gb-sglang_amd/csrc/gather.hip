@@ -38,12 +38,7 @@ struct Pools {
   const uint16_t* sm_k;  // [H, D] fp16, multiplied after the scale (identity in the served setup)
   const uint16_t* sm_v;
   int64_t ring_mask;
-  bool sm16;             // both smoothing tensors 16-byte aligned
 };
-
-bool sm_aligned(const void* sm_k, const void* sm_v) {
-  return ((reinterpret_cast<uintptr_t>(sm_k) | reinterpret_cast<uintptr_t>(sm_v)) & 15) == 0;
-}
 
 // rows per wavefront: 2 for the top-k gather (random rows: more wavefronts in flight), 4 for the whole-prefix
 // gather (streaming) -- 174.7 against 192 us and 1.55 against 1.69 ms per 12-layer step, the better of 2, 4 and 8
@@ -93,20 +88,6 @@ KVT_DEV uint4 dequant4(const Raw& r, const float m[8]) {   // ((b & 15) - 8) * s
   return make_uint4(bf16x2(x[0], x[1]), bf16x2(x[2], x[3]), bf16x2(x[4], x[5]), bf16x2(x[6], x[7]));
 }
 
-// 8 smoothing factors as fp32: one 16-byte load where the tensor is 16-byte aligned (sm16), else element loads (the
-// factors need only 2-byte alignment)
-KVT_DEV void load_sm(const uint16_t* p, bool sm16, float m[8]) {
-  if (sm16) {
-    const uint4 w = *reinterpret_cast<const uint4*>(p);
-    const uint32_t x[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) m[i] = f16_bits_to_f32((uint16_t)(x[i >> 1] >> (16 * (i & 1))));
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) m[i] = f16_bits_to_f32(p[i]);
-  }
-}
-
 // 16 bytes of an output row, non-temporal: the scratch is read by a later launch, and written through the caches as
 // ordinary stores it set the kernel's time (71,532 tokens, 188 MB moved: 53 us with plain stores, 31 us = 6.0 TB/s with
 // these; top-k selections of 16,408 rows 14.9 -> 14.6 us)
@@ -136,9 +117,14 @@ KVT_DEV void gather_rows(const Pools& P, const int64_t slot[ROWS], const int64_t
   const int U = H * CG;
   for (int u = lane; u < U; u += 64) {
     const int h = u / CG, cg = u - h * CG;
-    float mk[8], mv[8];   // once per unit
-    load_sm(P.sm_k + h * D + 8 * cg, P.sm16, mk);
-    load_sm(P.sm_v + h * D + 8 * cg, P.sm16, mv);
+    // once per unit, as element loads (the factors need only 2-byte alignment).  A branch to one 16-byte load where they
+    // are aligned made every row's loads wait for the factors: 12 pools of 71,532 tokens in turn 43 -> 62 us each.
+    float mk[8], mv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      mk[i] = f16_bits_to_f32(P.sm_k[h * D + 8 * cg + i]);
+      mv[i] = f16_bits_to_f32(P.sm_v[h * D + 8 * cg + i]);
+    }
     Raw rk[ROWS], rv[ROWS];
 #pragma unroll
     for (int j = 0; j < ROWS; ++j) {
