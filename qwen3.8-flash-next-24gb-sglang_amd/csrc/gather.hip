@@ -88,9 +88,15 @@ KVT_DEV uint4 dequant4(const Raw& r, const float m[8]) {   // ((b & 15) - 8) * s
   return make_uint4(bf16x2(x[0], x[1]), bf16x2(x[2], x[3]), bf16x2(x[4], x[5]), bf16x2(x[6], x[7]));
 }
 
-// 16 bytes of an output row, non-temporal: the scratch is read by a later launch, and written through the caches as
-// ordinary stores it set the kernel's time (71,532 tokens, 188 MB moved: 53 us with plain stores, 31 us = 6.0 TB/s with
-// these; top-k selections of 16,408 rows 14.9 -> 14.6 us)
+// 16 bytes of an output row, non-temporal.  The next launch reads the scratch, so what a store leaves in the caches counts
+// with the gather's own time.  Measured as a program gathers, 12 layers' pools in turn into one scratch (us per layer,
+// ordinary -> non-temporal stores): prefix of 60,000 tokens 38.0 -> 37.7, 20,480 tokens 16.3 -> 14.0, top-k 8 x 2,051 rows
+// 14.6 -> 12.9; with the attention of a dense chunk over each scratch the pair takes as long (60,000 x 1,024 queries 1,185 ->
+// 1,181, x 128 queries 218 -> 217, 20,480 x 128 queries 110 -> 110), with a launch that only streams the top-k scratch less
+// (32.5 -> 30.7).  A reader bound by the bytes of a large prefix scratch pays: non-temporal rows are not found in the
+// memory-side cache (60,000 x 16 queries 280 -> 286, sums over 71,532 rows 86.3 -> 92.9).  Gathers into a scratch of their
+// own each time gain most, since the output does not push the pools out of that cache (71,532 tokens 48.6 -> 31.1, repeated;
+// as long on a first pass).
 KVT_DEV void st_out(uint16_t* p, uint4 v) {
   typedef uint32_t u4v __attribute__((ext_vector_type(4)));
   __builtin_nontemporal_store((u4v){v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(p));
