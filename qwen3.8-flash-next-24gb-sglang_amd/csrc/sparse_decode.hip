@@ -729,7 +729,7 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     c_end = visible < (int64_t)A.topk ? (visible > 0 ? visible : 0) : (int64_t)A.topk;
   } else {
     qrow = b;
-    const int64_t vcount = A.all_columns != 0 ? L : x1 - x0;
+    const int64_t vcount = A.all_columns != 0 ? (int64_t)A.topk : x1 - x0;
     const int64_t span = (int64_t)kCols * (MULTI ? A.tiles : 1);
     c_begin = (int64_t)wx * span;
     const int64_t lim = vcount < (int64_t)A.topk ? vcount : (int64_t)A.topk;

@@ -88,3 +88,42 @@ def test_all_columns_equals_counted(kvt_pkg):
                                           **ring).cpu() for c in (cu, sa.ALL_COLUMNS)]
         assert torch.isnan(out[0][0]).all() and not torch.isnan(out[0][1:]).any()
         assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
+
+
+def test_all_columns_takes_every_column(kvt_pkg):
+    """ALL_COLUMNS attends a valid entry wherever it stands: rows whose valid entries come last, behind -1 padding, and
+    in between, at columns beyond the request's length (lengths 3 to 100 against 512 columns), equal the call whose
+    counts say all 512 columns, bit for bit, and the oracle; one tile per wavefront and several, merged in the launch
+    and by the combine."""
+    from kvtier import sparse_attn as sa
+    gen = torch.Generator().manual_seed(74)
+    R, slots, topk = 1024, 4096, 512
+    p = slot_pools(slots, R, 64, gen)
+    lens = torch.tensor([3, 40, 100, 100], dtype=torch.int32)
+    n = lens.numel()
+    idx = torch.full((n, topk), -1, dtype=torch.int32)
+    for b in range(n):
+        valid = torch.randperm(int(lens[b]), generator=gen).to(torch.int32)
+        at = torch.arange(topk - valid.numel(), topk) if b % 2 == 0 else torch.randperm(topk, generator=gen)[:valid.numel()]
+        idx[b, at] = valid
+    idx[3, idx[3] < 0] = 100   # (at the length: not attended)
+    r2t = torch.stack([torch.randperm(slots, generator=gen)[:100] for _ in range(n)]).to(torch.int32)
+    q = (torch.randn(n, HQ, D, generator=gen) / 4).to(torch.bfloat16)
+    exp = torch.empty(n, HQ, D)
+    gs = HQ // H
+    for b in range(n):
+        kk, vv = slot_rows("tiered", p, r2t[b, :int(lens[b])].long(), R, 64)
+        for h in range(H):
+            exp[b, h * gs:(h + 1) * gs] = ref.attention_rows(q[b, h * gs:(h + 1) * gs], kk[:, h:h + 1], vv[:, h:h + 1],
+                                                             D ** -0.5)
+    cu = (torch.arange(n + 1) * topk).to(torch.int32).to(dev)
+    a = pool_args("tiered", p, R, dev)
+    ring = {k: a[k] for k in a if k.startswith(("ring_", "owner"))}
+    for splits in (8, 3, 1):
+        for merge in ("launch", "combine"):
+            out = [sa.qwen_sparse_decode_attn(
+                q.to(dev), a["k_buf"], a["v_buf"], r2t.to(dev), torch.arange(n, device=dev), idx.to(dev), lens.to(dev), c, n,
+                topk, a["k_scale"], a["v_scale"], a["sm_k"], a["sm_v"], 4, splits=splits, merge=merge, **ring).cpu()
+                for c in (cu, sa.ALL_COLUMNS)]
+            assert torch.equal(out[0], out[1]), (splits, merge)
+            close(out[1], exp)
