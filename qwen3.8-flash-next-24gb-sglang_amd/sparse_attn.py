@@ -217,7 +217,33 @@ def qwen_sparse_kv_extraction_compact_triton(
 
 
 ALL_COLUMNS = object()   # as cu_k of qwen_sparse_decode_attn: column c counts whenever indices[b, c] < seq_lens[b]
-_MULTI_BLOCKS = 512   # blocks of a long-selection launch: one per resident slot, 2 per CU (256 VGPRs)
+_MULTI_BLOCKS = 512   # resident slots of a long-selection launch: 2 blocks per CU (256 VGPRs)
+
+
+def _decode_splits(batch: int, heads: int, topk: int) -> int:
+    """Column splits per (request, KV head) of a sparse decode launch: 64 columns per block (a 16-column tile per
+    wavefront) while the launch holds at most 1,024 such blocks.  Longer selections take as many splits as fit the
+    resident slots in one round, each of the same number of tiles per wavefront: a round begun for a few blocks costs
+    as much as a full one.  Beyond 256 (request, KV head) pairs two splits no longer fit and the launch takes about
+    512 blocks, rounded up.
+
+    Measured (us per layer with the combine, 24 / 2 heads, top-k x requests):
+    * one round against the next larger count: 1,024 x 48 4 splits (384 blocks) 28.1, 6 (576) 36.9; 512 x 96 2 (384)
+      29.0, 3 (576) 35.2; 1,024 x 70 3 (420) 31.4, 4 (560) 44.1; 2,051 x 100 2 (400) 63.9, 3 (600) 73.9; dense positions
+      4 x 65,536 512 blocks 51, 768 80; 6 x 65,536 492 blocks 72.8, 516 107.6 (but with 4 of the 6 requests at 100
+      positions, whose blocks are empty, 56.5 and 55.2).
+    * beyond 256 pairs: 2,051 x 150 1 split (300 blocks) 106.1, 2 (600) 104.3; 1,024 x 200 1 (400) 60.2, 2 (800) 71.2; the
+      single split's sums are twice as long (error against 64 bits 1.29e-6 and 1.17e-6, against 1.15e-6 and 1.04e-6).
+    * the line at 1,024: 2,051 x 15 (990 blocks) one tile 23.6, two 21.7; x 16 (1,056) one tile 24.4, three 23.3; 1,024 x 32
+      (1,024) 24.5, four 23.2; x 33 (1,056) 25.1, three 26.1.  With 16 / 2 heads 20.9 / 20.1, 21.0 / 21.7, 21.2 / 21.6 and
+      21.9 / 23.3.  The two kernels cross near it; short selections of many requests (512 x 64: 33.2, two tiles 24.3)
+      would cross earlier."""
+    pairs, tiles64 = batch * heads, (topk + 63) // 64
+    if pairs * tiles64 <= 1024:
+        return tiles64
+    fit = _MULTI_BLOCKS // pairs
+    tiles = -(-tiles64 // fit) if fit >= 2 else -(-pairs * tiles64 // _MULTI_BLOCKS)   # per wavefront
+    return -(-tiles64 // tiles)
 
 
 def qwen_sparse_decode_attn(
@@ -276,14 +302,7 @@ def qwen_sparse_decode_attn(
         return out
     _lib.require_device(q, k, v, req_to_token, indices, out)
     scale = float(dim ** -0.5) if scale is None else float(scale)
-    # blocks of 64 selected columns (a 16-column tile per wavefront) while the launch holds at most 1,024 of them;
-    # longer selections take `tiles` tiles per wavefront in about one block per resident slot (2 per CU: 55 us
-    # for 4 x 65,536 dense positions, against 63 us at 1,024 blocks and 80 us at 768), each
-    # partial then covering 64 x tiles columns
-    tiles64 = (int(topk) + 63) // 64
-    blocks = batch * heads * tiles64
-    tiles = 1 if blocks <= 1024 else -(-blocks // _MULTI_BLOCKS)
-    n_splits = -(-tiles64 // tiles) if splits is None else int(splits)
+    n_splits = _decode_splits(batch, heads, int(topk)) if splits is None else int(splits)
     assert n_splits >= 1
     ws = workspace if workspace is not None else {}
     need = batch * heads * n_splits * (Hq // heads)

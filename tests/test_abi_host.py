@@ -264,3 +264,30 @@ def test_sparse_decode_merge_arguments_refused(kvt_pkg):
                dict(out_f32=P + 4), dict(n_splits=(1 << 31) // ((Hq // H) * D * 4))):
         with pytest.raises(ValueError):
             call(**kw)
+
+
+@pytest.mark.parametrize("batch,topk", [(1, 1), (8, 2051), (16, 2048), (16, 2051), (33, 1024), (44, 1024), (48, 1024), (70, 1024),
+                                        (96, 512), (100, 2051), (128, 2051), (150, 2051), (300, 2051), (4, 65536), (6, 8192)])
+def test_sparse_decode_blocks_fit_one_round(kvt_pkg, monkeypatch, batch, topk):
+    """A sparse decode launch of more than one tile per wavefront (2 KV heads) begins no second round of resident
+    blocks (512 slots) up to 256 (request, KV head) pairs, and its splits are of equal tiles, none without columns; up to 1,024 blocks of 64 columns it takes one tile per wavefront.  The launch is intercepted:
+    the split count shows in the workspace."""
+    from kvtier import _lib, sparse_attn as sa
+    H, D, slots = 2, 256, 64
+    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
+    monkeypatch.setattr(_lib, "stream", lambda *a: 0)
+    monkeypatch.setattr(_lib, "call", lambda *a: None)
+    pool = [torch.zeros(slots, H, D, dtype=torch.int8)] * 2 + [torch.zeros(slots, H, 4, dtype=torch.float16)] * 2
+    idx = torch.zeros(1, topk, dtype=torch.int32).expand(batch, topk)
+    ws = {}
+    sa.qwen_sparse_decode_attn(torch.zeros(batch, 2, D, dtype=torch.bfloat16), pool[0], pool[1],
+                               torch.zeros(batch, 64, dtype=torch.int32), torch.zeros(batch, dtype=torch.int64), idx,
+                               torch.ones(batch, dtype=torch.int32), torch.zeros(batch + 1, dtype=torch.int32), batch,
+                               topk, pool[2], pool[3], kv_bits=8, workspace=ws)
+    splits, tiles64 = ws["sparse_o"].numel() // (batch * H * D), -(-topk // 64)
+    if batch * H * tiles64 <= 1024:
+        assert splits == tiles64
+    else:
+        tiles = -(-tiles64 // splits)
+        assert batch * H > 256 or batch * H * splits <= 512
+        assert splits == -(-tiles64 // tiles)
