@@ -93,10 +93,13 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def stream() -> int:
-    """The current device's current stream as a raw handle (torch's raw-handle query; the Stream object around it cost
-    about 1 us of each eager call)."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+def stream(device: Optional[int] = None) -> int:
+    """The current stream of a device (index; default the current device) as a raw handle: by torch's raw-handle query,
+    a private name of torch, where this torch has it, else through the public Stream object (2.8 us a call
+    against 0.33)."""
+    idx = torch.cuda.current_device() if device is None else device
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(idx) if raw is not None else torch.cuda.current_stream(idx).cuda_stream
 
 
 def require_device(*tensors: Optional[torch.Tensor]) -> None:

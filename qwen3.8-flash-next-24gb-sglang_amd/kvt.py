@@ -719,7 +719,7 @@ def prefill_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     streams get their own, so launches that may overlap never share counters.  (Allocate it before a graph capture:
     capture records on a side stream, which then owns a workspace of its own.)"""
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    key = (idx, torch._C._cuda_getCurrentRawStream(idx))
+    key = (idx, _lib.stream(idx))
     ws = _prefill_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1), dtype=torch.uint8, device=device)

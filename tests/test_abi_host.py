@@ -3,6 +3,7 @@ signatures cover exactly those, and the host logic (guards, env parsing, page al
 reference's (patches/kv_tiers.py:91-100, :176-220; gemv/test_kv_tiers.py:463-473, :539-551).  No kernel runs."""
 import ctypes
 import os
+import types
 
 import pytest
 import torch
@@ -291,3 +292,19 @@ def test_sparse_decode_blocks_fit_one_round(kvt_pkg, monkeypatch, batch, topk):
         tiles = -(-tiles64 // splits)
         assert batch * H > 256 or batch * H * splits <= 512
         assert splits == -(-tiles64 // tiles)
+
+
+def test_stream_handle_without_the_private_query(kvt_pkg, monkeypatch):
+    """The stream handle comes from torch's private raw-handle query where torch has it and from the public Stream
+    object where it does not, for the current device and for a given one; the cached prefill workspace is keyed by it."""
+    from kvtier import _lib, kvt
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: types.SimpleNamespace(cuda_stream=100 + (3 if d is None else d)))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 200 + d, raising=False)
+    assert (_lib.stream(), _lib.stream(1)) == (203, 201)
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert (_lib.stream(), _lib.stream(1)) == (103, 101)
+    monkeypatch.setattr(kvt, "_prefill_ws", {})
+    monkeypatch.setattr(torch, "zeros", lambda n, **k: types.SimpleNamespace(numel=lambda: n))
+    kvt.prefill_workspace(torch.device("cuda", 1), 64)
+    assert list(kvt._prefill_ws) == [(1, 101)]
