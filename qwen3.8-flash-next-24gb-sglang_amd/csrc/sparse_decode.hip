@@ -415,7 +415,7 @@ KVT_DEV uint32_t resolve_tile(const SparseArgs& A, int64_t c0, int64_t c_end, co
   return word;
 }
 
-// LDS of a block: one tile buffer per wavefront (K rows until S is formed, then V rows; 42 KB per block), after the
+// LDS of a block: one tile buffer per wavefront (K rows until S is formed, then V rows), after the
 // tiles the same space holds the merge of the 4 wavefronts; and the group's q heads, bf16 (zero beyond gs)
 template <int CAP>
 struct BlockLds {
@@ -429,8 +429,11 @@ struct BlockLds {
   int ones[kWaves];            // wavefront w's smoothing factors are all 1
   int last;                    // decode merged in the launch: this block counted last for its (request, KV head)
 };
-constexpr int kRowCols = 4096;   // prefill rows: selected columns resolved per pass (74 KB of LDS per block)
-constexpr int kMultiCols = 1024; // decode blocks of several tiles per wavefront (50 KB of LDS per block)
+constexpr int kRowCols = 4096;   // prefill rows: selected columns resolved per pass
+constexpr int kMultiCols = 1024; // decode blocks of several tiles per wavefront
+// LDS per block, of 160 KB a CU: 3 one-tile blocks, 2 of the others (their registers allow no third)
+static_assert(sizeof(BlockLds<1>) == 43512 && sizeof(BlockLds<kMultiCols>) == 47604 && sizeof(BlockLds<kRowCols>) == 59892,
+              "LDS per block");
 
 // The selected columns [k0, k1) (at most CAP) of a block's query row, resolved by all its threads
 // together into the column table and partitioned by tier: ring (INT8) rows to cols[0 .. nh), INT4 rows from the end
@@ -711,9 +714,11 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     }
   };
   if constexpr (!ROWS) load_q(b);
-  // the head's smoothing factors, 2 per thread: K's, then V's (an absent tensor: all 1)
+  // the head's smoothing factors, 2 per thread: K's, then V's (an absent tensor: all 1).  The tensors need only 2-byte
+  // alignment.
+  typedef uint32_t u32_at2 __attribute__((aligned(2)));
   const uint16_t* smp = threadIdx.x < kD / 2 ? A.sm_k : A.sm_v;
-  const uint32_t smw = smp != nullptr ? reinterpret_cast<const uint32_t*>(smp + h * kD)[threadIdx.x & (kD / 2 - 1)]
+  const uint32_t smw = smp != nullptr ? reinterpret_cast<const u32_at2*>(smp + h * kD)[threadIdx.x & (kD / 2 - 1)]
                                       : 0x3c003c00u;
   __builtin_amdgcn_sched_barrier(0);
   const int64_t req = idx_value(wreq), x0 = idx_value(w0), x1 = idx_value(w1), L = len;
@@ -756,8 +761,8 @@ KVT_DEV void sparse_attn_block(const SparseArgs& A, BlockLds<CAP>& S) {
     const int hq = i / (kD / 8), ch = i - hq * (kD / 8);
     *reinterpret_cast<uint4*>(&qs[hq * kKPitch + 8 * ch]) = qv[k];
   }
-  PoolRsrc P;
-  {
+  PoolRsrc P;   // both tiers' descriptors, for the one-tile blocks (a column table's loops build one tier's each)
+  if constexpr (CAP == 1) {
     const uint32_t n8 = A.rows8 * (uint32_t)H * kD, n4 = A.rows4 * (uint32_t)H * (kD / 2);
     const uint32_t s8 = A.rows8 * (uint32_t)H * (kD / G8) * 2, s4 = A.rows4 * (uint32_t)H * (kD / kG4) * 2;
     P.k8 = rsrc(KIND == 2 ? (const void*)A.rk : A.k, KIND == 1 ? 0u : n8);
