@@ -134,7 +134,7 @@ int kvt_compact_gather(int kind, const void* k, const void* v, const void* k_sca
  * block of a (request, KV head) that counts last merges its n_splits partials in split order and writes out_f32 or
  * out_bf16 (exactly one; [batch, Hq, D] rows with batch stride out_stride_b >= Hq * D, a multiple of 8, 16-byte
  * aligned); calls sharing the counters and
- * partials must not overlap.  Faster than the combine launch for few splits (<= 8), slower for many: one block
+ * partials must not overlap.  Faster than the combine launch for few splits (<= 4, with many requests <= 7), slower for many: one block
  * reads all of a (request, KV head)'s partials.  cu_k NULL: every column counts (column c of request b is attended
  * when 0 <= indices[b][c] < seq_lens[b]).  A request with no attended column comes out
  * NaN (0/0).  n_splits >= 1; Hq / H <= 16, D = 256.  Kinds and buffers as kvt_compact_gather; pool_rows = rows of k / v (byte offsets

@@ -228,15 +228,15 @@ def _decode_splits(batch: int, heads: int, topk: int) -> int:
     512 blocks, rounded up.
 
     Measured (us per layer with the combine, 24 / 2 heads, top-k x requests):
-    * one round against the next larger count: 1,024 x 48 4 splits (384 blocks) 28.1, 6 (576) 36.9; 512 x 96 2 (384)
-      29.0, 3 (576) 35.2; 1,024 x 70 3 (420) 31.4, 4 (560) 44.1; 2,051 x 100 2 (400) 63.9, 3 (600) 73.9; dense positions
+    * one round against the next larger count: 1,024 x 48 4 splits (384 blocks) 26.1, 6 (576) 34.2; 512 x 96 2 (384)
+      27.3, 3 (576) 33.8; 1,024 x 70 3 (420) 29.6, 4 (560) 41.0; 2,051 x 100 2 (400) 62.1, 3 (600) 70.0; dense positions
       4 x 65,536 512 blocks 51, 768 80; 6 x 65,536 492 blocks 72.8, 516 107.6 (but with 4 of the 6 requests at 100
       positions, whose blocks are empty, 56.5 and 55.2).
-    * beyond 256 pairs: 2,051 x 150 1 split (300 blocks) 106.1, 2 (600) 104.3; 1,024 x 200 1 (400) 60.2, 2 (800) 71.2; the
+    * beyond 256 pairs: 2,051 x 150 1 split (300 blocks) 104.6, 2 (600) 101.4; 1,024 x 200 1 (400) 59.0, 2 (800) 68.1; the
       single split's sums are twice as long (error against 64 bits 1.29e-6 and 1.17e-6, against 1.15e-6 and 1.04e-6).
-    * the line at 1,024: 2,051 x 15 (990 blocks) one tile 23.6, two 21.7; x 16 (1,056) one tile 24.4, three 23.3; 1,024 x 32
-      (1,024) 24.5, four 23.2; x 33 (1,056) 25.1, three 26.1.  With 16 / 2 heads 20.9 / 20.1, 21.0 / 21.7, 21.2 / 21.6 and
-      21.9 / 23.3.  The two kernels cross near it; short selections of many requests (512 x 64: 33.2, two tiles 24.3)
+    * the line at 1,024: 2,051 x 15 (990 blocks) one tile 23.4, two 21.6; x 16 (1,056) one tile 24.4, three 23.3; 1,024 x 32
+      (1,024) 23.9, four 22.3; x 33 (1,056) 24.8, three 23.5.  With 16 / 2 heads 20.6 / 20.4, 21.0 / 21.8, 21.2 / 21.3 and
+      21.5 / 22.2.  The two kernels cross near it; short selections of many requests (512 x 64: 26.9, two tiles 22.3)
       would cross earlier."""
     pairs, tiles64 = batch * heads, (topk + 63) // 64
     if pairs * tiles64 <= 1024:
@@ -258,8 +258,11 @@ def qwen_sparse_decode_attn(
     block of a (request, KV head) that finishes last merges the column splits inside the launch (counters in the
     workspace: calls sharing a workspace must not overlap); merge="combine": the splits go through
     kvt_decode_combine, a second launch; merge="auto" (default): in the launch for at most 8 splits per (request, KV
-    head), where it is the faster of the two (one block then reads at most 8 partials of up to 16 x 1 KB), else the
-    combine launch, whose blocks (one per request, q head and slice of dims) read the partials side by side.
+    head), where one block reads at most 8 partials of up to 16 x 1 KB, else the combine launch, whose blocks (one per
+    request, q head and slice of dims) read the partials side by side.  In the launch against the combine, us per layer
+    (24 / 2 heads): 1 split 11.5 / 13.8 (32 requests), 4 13.8 / 15.0 (32) and 12.0 / 11.9 (8), 7 29.9 / 31.0 (32, several
+    tiles) and 13.2 / 12.0 (8), 8 18.2 / 17.3 (32) and 13.6 / 12.0 (8), 9 27.6 / 27.2 (24), 11 24.5 / 23.5 (16), 33 28.7 / 16.3
+    (8): few requests would take the combine from 4 splits on.
 
     q: bf16 [batch, Hq, D]; the pool/ring/owner/scale arguments as the compact gather; cu_k: the valid counts'
     prefix sum (qwen_sparse_fa2_cu_seqlens_triton), or ALL_COLUMNS.  Column c of request b is attended when c < cu_k[b+1] - cu_k[b]
