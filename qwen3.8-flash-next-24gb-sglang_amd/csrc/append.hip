@@ -7,9 +7,9 @@
 // division on the common path: scales from a * fl(1/qmax) and codes from x * rcp(s), each checked against the
 // rounding ties it could get wrong, with the IEEE division for the lanes that are close to one.
 //
-//   kvt_quant_store_tiered  dual write (patches/kv_tiers.py:272-443): the owner stamp (inside the write for up to
-//                           kScanTokens tokens, a launch before it for more), the INT8 ring row (owner only) and the
-//                           INT4 pool row (always).
+//   kvt_quant_store_tiered  dual write (patches/kv_tiers.py:272-443): the owner stamp (inside the write for short calls, see
+//                           kScanTokens, a launch before it for others), the INT8 ring row (owner only) and the INT4
+//                           pool row (always).
 //   kvt_quant_store_int8    INT8-G quant + scatter (patches/kv_int8.py:281-362, with the fp16-max clamp).
 //   kvt_quant_store_int4    INT4-G32 quant + nibble pack + scatter (patches/kv_int4.py:289-393).
 //   kvt_page_table_update   writes (seq, logical page) -> physical page entries before an evicting append.
@@ -281,24 +281,25 @@ __global__ void __launch_bounds__(256) stamp_owner_kernel(const void* loc, int l
 // The owner stamp inside the dual write.  Every wavefront finds the winner of its own ring row among the N slots of
 // the call by itself: the last token whose slot falls in that ring row (any rule that all wavefronts share gives one
 // winner per row).  So nothing is read that another wavefront writes, and the stamp needs no launch of its own.  The
-// scan's loads go out together with the inputs'.  Returns the ring row's new owner word; *last: the winner's token.
-template <int LANES>
-KVT_DEV int32_t scan_owner(const void* loc, int loc64, uint32_t N, int64_t slot, int64_t ring_mask, int lane,
-                           uint32_t* last) {
+// scan's loads go out together with the inputs'; all 64 lanes scan (those that hold no channel of the row as well),
+// and the two widths of the slots have a loop each (a choice per load made each wait for the one before).  Returns the
+// ring row's new owner word; *last: the winner's token.
+template <typename T>
+KVT_DEV int32_t scan_slots(const T* loc, uint32_t N, int64_t slot, int64_t ring_mask, int lane, uint32_t* last) {
   constexpr int kAhead = 4;   // slots per lane in flight
   uint32_t win = 0;
   int32_t word = (int32_t)slot;   // (the row's own token matches, so some slot is always taken below)
-  for (uint32_t b = 0; b < N; b += kAhead * LANES) {
-    int64_t s[kAhead];
+  for (uint32_t b = 0; b < N; b += kAhead * 64) {
+    T s[kAhead];
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) s[j] = load_loc(loc, loc64, min(b + (uint32_t)(j * LANES + lane), N - 1));
+    for (int j = 0; j < kAhead; ++j) s[j] = loc[min(b + (uint32_t)(j * 64 + lane), N - 1)];
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) {
-      const uint32_t i = b + (uint32_t)(j * LANES + lane);
-      const uint64_t m = __builtin_amdgcn_ballot_w64(i < N && ((s[j] ^ slot) & ring_mask) == 0);
+      const uint32_t i = b + (uint32_t)(j * 64 + lane);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(i < N && (((int64_t)s[j] ^ slot) & ring_mask) == 0);
       if (m != 0) {
         const int at = 63 - __builtin_clzll(m);
-        win = b + (uint32_t)(j * LANES + at);
+        win = b + (uint32_t)(j * 64 + at);
         word = __builtin_amdgcn_readlane((int32_t)s[j], at);
       }
     }
@@ -306,11 +307,18 @@ KVT_DEV int32_t scan_owner(const void* loc, int loc64, uint32_t N, int64_t slot,
   *last = win;
   return word;
 }
+KVT_DEV int32_t scan_owner(const void* loc, int loc64, uint32_t N, int64_t slot, int64_t ring_mask, int lane,
+                           uint32_t* last) {
+  return loc64 ? scan_slots(reinterpret_cast<const int64_t*>(loc), N, slot, ring_mask, lane, last)
+               : scan_slots(reinterpret_cast<const int32_t*>(loc), N, slot, ring_mask, lane, last);
+}
 
-// Calls of at most this many tokens stamp inside the dual write, longer ones in a launch before it: the scan costs
-// every wavefront N slot reads, the launch 1.4 us whatever N (12 layers, two launches each against one: 56.7 -> 40.5 us
-// for 8 tokens, 62.0 -> 45.2 for 256, 68.1 -> 54.8 for 512, 78.9 -> 72.3 for 1,024, but 90.9 -> 111.6 for 2,048).
-constexpr int64_t kScanTokens = 1024;
+// Calls of at most kScanTokens tokens stamp inside the dual write, as long as the scan reads at most kScanReads slots in
+// all (every wavefront, one per token and head, reads N); others in a launch before it, which takes 1.2-1.4 us whatever N
+// until the chip is full.  Launch against scan, us per call (D = 256, int64 slots): 2 heads 8 tokens 4.8 / 3.4, 256
+// 5.3 / 3.9, 1,024 6.4 / 5.6, 1,536 7.0 / 7.1, 2,048 7.6 / 9.1; 8 heads 640 (3.3 M reads) 7.2 / 6.8, 768 (4.7 M) 7.5 / 7.3, 896 (6.4 M)
+// 8.1 / 8.6; 16 heads 512 (4.2 M) 8.4 / 7.6, 640 (6.6 M) 9.3 / 9.6.
+constexpr int64_t kScanTokens = 1024, kScanReads = 1 << 22;
 
 // MODE 0: tiered dual write after an owner stamp launch; 1: INT8 only (ring buffers are the pool); 2: INT4 only; 3:
 // tiered dual write with the stamp inside.  The row's slot index (and in MODE 0 the owner word of its ring row) are
@@ -324,8 +332,12 @@ __global__ void __launch_bounds__(256) quant_store_kernel(
   const int lane = threadIdx.x & 63;
   uint32_t t;
   int h;
-  if (!wave_row(NH, H, &t, &h) || lane >= D / 4) return;
-  const int c0 = 4 * lane;
+  if (!wave_row(NH, H, &t, &h)) return;
+  const bool live = lane < D / 4;   // this lane holds channels of the row
+  if constexpr (MODE != 3) {
+    if (!live) return;
+  }
+  const int c0 = 4 * (live ? lane : D / 4 - 1);   // (MODE 3 with D < 256: the others reread the last channels)
   const In4 rk_in = load4_raw<DT, LM>(kin, t, h, c0, sm_k_inv, D);
   const In4 rv_in = load4_raw<DT, LM>(vin, t, h, c0, sm_v_inv, D);
   __builtin_amdgcn_sched_barrier(0);
@@ -337,9 +349,10 @@ __global__ void __launch_bounds__(256) quant_store_kernel(
   }
   if constexpr (MODE == 3) {
     uint32_t last;
-    const int32_t word = scan_owner<D / 4>(loc, loc64, NH / (uint32_t)H, slot, ring_mask, lane, &last);
+    const int32_t word = scan_owner(loc, loc64, NH / (uint32_t)H, slot, ring_mask, lane, &last);
     hot = (int64_t)word == slot;
     if (t == last && h == 0 && lane == 0) owner[slot & ring_mask] = word;
+    if (!live) return;
   }
   __builtin_amdgcn_sched_barrier(0);
   float xk[4], xv[4];
@@ -603,7 +616,7 @@ int kvt_quant_store_tiered(const void* k, const void* v, int dtype, int64_t sk_n
         (uint8_t*)v_buf, (uint16_t*)k_scale, (uint16_t*)v_scale, (int8_t*)ring_k, (int8_t*)ring_v, (uint16_t*)ring_ks,
         (uint16_t*)ring_vs, (int32_t*)owner, (const uint16_t*)sm_k_inv, (const uint16_t*)sm_v_inv, ring_mask, st);
   };
-  if (N <= kScanTokens) return store(std::integral_constant<int, 3>{});
+  if (N <= kScanTokens && N * N * H <= kScanReads) return store(std::integral_constant<int, 3>{});
   const unsigned sblocks = (unsigned)((N + 255) / 256);
   hipLaunchKernelGGL(stamp_owner_kernel, dim3(sblocks), dim3(256), 0, st, loc, loc_is_int64, N, (int32_t*)owner,
                      ring_mask);

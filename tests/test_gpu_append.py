@@ -203,6 +203,44 @@ def test_tiered_stamp_inside_the_write(kvt_pkg, n, loc_dtype, dt, g8):
         assert (c[4 + t][~written] == fill).all() and (c[6 + t][~written] == scale).all()
 
 
+@pytest.mark.parametrize("n,heads,dim,loc_dtype", [(63, 2, 64, torch.int64), (257, 3, 128, torch.int32),
+                                                   (724, 8, 128, torch.int64), (725, 8, 128, torch.int32),
+                                                   (1024, 4, 256, torch.int32), (1024, 5, 256, torch.int64)])
+def test_tiered_stamp_line_by_slot_reads(kvt_pkg, n, heads, dim, loc_dtype):
+    """The stamp stands inside the write up to 1,024 tokens and tokens^2 * heads <= 2^22 slot reads, in a launch before it
+    beyond: both sides of the line, and rows of fewer channels than a wavefront's lanes hold (all lanes scan).  One
+    winner per contested ring row, its row and every INT4 row bit-exact."""
+    from kvtier import sparse_attn as sa
+    gen = torch.Generator().manual_seed(80 + n)
+    rings, slots = 2048, 8192
+    k, v = [(torch.randn(n, heads, dim, generator=gen) * 3).to(torch.bfloat16) for _ in range(2)]
+    i = torch.randperm(n, generator=gen)                       # tokens 2 j and 2 j + 1 (in some order) share ring row j
+    loc = (torch.randint(0, 4, (n,), generator=gen)[i // 2] + i % 2) % 4 * rings + i // 2
+    b = [torch.zeros(slots, heads, dim // 2, dtype=torch.uint8, device=dev) for _ in range(2)]
+    b += [torch.zeros(slots, heads, dim // 32, dtype=torch.float16, device=dev) for _ in range(2)]
+    b += [torch.full((rings, heads, dim), 0x33, dtype=torch.int8, device=dev) for _ in range(2)]
+    b += [torch.full((rings, heads, dim // 64), 7.0, dtype=torch.float16, device=dev) for _ in range(2)]
+    b += [torch.full((rings,), -1, dtype=torch.int32, device=dev)]
+    ones = torch.ones(heads, dim, dtype=torch.float16, device=dev)
+    sa.quant_store_kv_tiered(k.to(dev), v.to(dev), loc.to(loc_dtype).to(dev), *b, ones, ones, rings - 1)
+    torch.cuda.synchronize()
+    c = _cpu(b)
+    owner = c[8].long()
+    written = torch.zeros(rings, dtype=torch.bool)
+    written[loc % rings] = True
+    at = torch.full((slots,), -1, dtype=torch.long)
+    at[loc] = torch.arange(n)
+    own = owner[written]
+    assert torch.equal(owner >= 0, written) and (at[own] >= 0).all()
+    assert torch.equal(own % rings, torch.nonzero(written).flatten())
+    for t, x in enumerate((k, v)):
+        p4, s4 = ref.quant4(x)
+        assert torch.equal(c[t][loc], p4) and torch.equal(c[2 + t][loc], s4)
+        q8, s8 = ref.quant8(x)
+        assert torch.equal(c[4 + t][own % rings], q8[at[own]]) and torch.equal(c[6 + t][own % rings], s8[at[own]])
+        assert (c[4 + t][~written] == 0x33).all() and (c[6 + t][~written] == 7.0).all()
+
+
 def test_fp16_max_clamp_writers(kvt_pkg):
     """1e6 / bf16-max groups: ring and INT4 scales 65504, codes bit-exact vs the clamped references
     (gemv/test_kv_tiers.py:412-436)."""
