@@ -17,6 +17,8 @@
 //   kvt_sparse_cu_seqlens  valid top-k counts and their prefix sum, the offsets kvt_compact_gather packs at (the
 //                       upstream qwen_sparse_fa2_cu_seqlens_triton the reference calls first, gemv/test_kv_tiers.py:297-301)
 
+#include <type_traits>
+
 #include "kvt_common.h"
 
 using namespace kvt;
@@ -229,19 +231,67 @@ bool aligned_args(int kind, const void* k, const void* v, const void* rk, const 
 
 
 // counts[b] = #{c < topk : 0 <= indices[b * idx_stride + c] < seq_lens[b]}; cu_k[0] = 0, cu_k[b + 1] = counts[0] + ..
-// + counts[b].  One block of kCuThreads, kCuThreads rows at a time: a row's columns go to one wavefront, or to several
-// where there are more wavefronts than rows, in chunks of 64 kCuAhead columns whose loads are in flight together (the
-// launch is a few dependent memory rounds long: 8 rows of 2,051 columns took 13.7 us with one load per round and one
-// wavefront per row, 7.0 us now); then the block scans the chunk's counts in LDS (Hillis-Steele, double-buffered)
-// and adds the running total of the earlier chunks.
-constexpr int kCuAhead = 16;
+// + counts[b].  One block of kCuThreads, kCuThreads rows at a time.  The launch is a few dependent memory rounds long, so
+// a wavefront keeps up to 16 loads in flight: the chunks of 64 columns of one row (1, 2, 4, 8 or 16, to a power of two), or
+// of as many rows as that leaves room for where there are that many rows for every wavefront; where there are fewer
+// rows than wavefronts, a row goes to several.  us with one load per round and a wavefront per row / 16 loads of one row
+// at a time / as it is: 8 x 64 columns 3.3 / 4.6 / 3.3, 8 x 2,051 7.1 / 5.7 / 5.6, 64 x 512 8.8 / 10.2 / 6.4, 256 x 64 9.3 /
+// 30.9 / 7.0, 1,024 x 512 92.6 / 113 / 47.0, 2,100 x 130 95 / 231 / 60 (worst against the first: 17 x 65 3.8 / 5.0 / 4.1).
+// Then the block scans the chunk's counts in LDS (Hillis-Steele, double-buffered) and adds the running total of the
+// earlier chunks.
 constexpr int kCuThreads = 1024;
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// Adds to buf[r .. r + G - 1] (rows past nrows left out) the valid entries of rows r0 + r .. in chunks of 64 A columns,
+// from column c0 on, `step` apart.
+template <int G, int A>
+KVT_DEV void count_rows(const int32_t* seq_lens, const int32_t* indices, int64_t idx_stride, int r0, int r, int nrows,
+                        int64_t c0, int64_t step, int topk, int lane, int32_t* buf) {
+  const int32_t* row[G];
+  int64_t L[G];
+  int n[G];   // A 1: the wavefront's count, else this lane's
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int b = r0 + (r + g < nrows ? r + g : nrows - 1);
+    L[g] = seq_lens[b];
+    row[g] = indices + (int64_t)b * idx_stride;
+    n[g] = 0;
+  }
+  for (; c0 < topk; c0 += step) {
+    int32_t p[G][A];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int j = 0; j < A; ++j) {   // (past the end: the last column, not counted)
+        const int64_t c = c0 + 64 * j + lane;
+        p[g][j] = row[g][c < topk ? c : topk - 1];
+      }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int j = 0; j < A; ++j) {
+        const bool valid = c0 + 64 * j + lane < topk && p[g][j] >= 0 && (int64_t)p[g][j] < L[g];
+        n[g] += A == 1 ? __popcll(__builtin_amdgcn_ballot_w64(valid)) : (valid ? 1 : 0);
+      }
+  }
+  if constexpr (A > 1) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int g = 0; g < G; ++g) n[g] += __shfl_xor(n[g], o, 64);
+  }
+  int mine = 0;
+#pragma unroll
+  for (int g = 0; g < G; ++g) mine = lane == g ? n[g] : mine;
+  if (lane < G && r + lane < nrows) atomicAdd(&buf[r + lane], mine);
+}
 
 __global__ void __launch_bounds__(kCuThreads) cu_seqlens_kernel(const int32_t* seq_lens, const int32_t* indices,
                                                                  int64_t idx_stride, int32_t* counts, void* cu_k,
                                                                  int cu_is_int64, int batch, int topk) {
   __shared__ int32_t buf[2][kCuThreads];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wave = wave_id();
   constexpr int kW = kCuThreads / 64;
   auto put = [&](int64_t i, int64_t v) {
     if (cu_is_int64) ((int64_t*)cu_k)[i] = v;
@@ -253,25 +303,29 @@ __global__ void __launch_bounds__(kCuThreads) cu_seqlens_kernel(const int32_t* s
     const int nrows = min(kCuThreads, batch - r0);
     buf[0][t] = 0;
     __syncthreads();
-    const int split = nrows < kW ? kW / nrows : 1;   // wavefronts per row
-    for (int item = wave; item < nrows * split; item += kW) {
-      const int r = item / split, b = r0 + r;
-      const int64_t L = seq_lens[b];
-      const int32_t* row = indices + (int64_t)b * idx_stride;
-      int n = 0;
-      for (int64_t c0 = (int64_t)(item - r * split) * 64 * kCuAhead; c0 < topk; c0 += (int64_t)split * 64 * kCuAhead) {
-        int32_t p[kCuAhead];
-#pragma unroll
-        for (int j = 0; j < kCuAhead; ++j) {   // (past the end: the last column, not counted)
-          const int64_t c = c0 + 64 * j + lane;
-          p[j] = row[c < topk ? c : topk - 1];
-        }
-#pragma unroll
-        for (int j = 0; j < kCuAhead; ++j) n += (c0 + 64 * j + lane < topk && p[j] >= 0 && (int64_t)p[j] < L) ? 1 : 0;
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-      if (lane == 0) atomicAdd(&buf[0][r], n);
+    int sh = 0;   // 2^sh wavefronts per row
+    while (nrows << (sh + 1) <= kW) ++sh;
+    const auto count = [&](auto g, auto a) {
+      constexpr int G = decltype(g)::value, A = decltype(a)::value;
+      for (int r = (wave >> sh) * G; r < nrows; r += (kW >> sh) * G)
+        count_rows<G, A>(seq_lens, indices, idx_stride, r0, r, nrows, (int64_t)(wave & ((1 << sh) - 1)) * 64 * A,
+                         (int64_t)(64 * A) << sh, topk, lane, buf[0]);
+    };
+    const int share = (topk - 1) >> sh;   // columns per wavefront
+    if (share < 64) {
+      if (nrows >= 8 * kW) count(Int<16>{}, Int<1>{});
+      else count(Int<1>{}, Int<1>{});
+    } else if (share < 256 && nrows >= 4 * kW) {
+      count(Int<4>{}, Int<4>{});
+    } else if (share < 128) {
+      count(Int<1>{}, Int<2>{});
+    } else if (share < 256) {
+      count(Int<1>{}, Int<4>{});
+    } else if (share < 512) {
+      if (nrows >= 2 * kW) count(Int<2>{}, Int<8>{});
+      else count(Int<1>{}, Int<8>{});
+    } else {
+      count(Int<1>{}, Int<16>{});
     }
     __syncthreads();
     int cur = 0;

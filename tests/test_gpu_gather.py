@@ -363,3 +363,12 @@ def test_cu_seqlens_kernel(kvt_pkg, batch, topk, cu64, shared):
     assert torch.equal(cu.cpu()[:batch + 1].to(torch.int32), want)
     assert torch.equal(counts.cpu()[:batch], (want[1:] - want[:-1]))
     assert bool((cu.cpu()[batch + 1:] == -7).all()) and bool((counts.cpu()[batch:] == -7).all())
+
+
+@pytest.mark.parametrize("batch,topk", [(2, 64), (15, 65), (9, 600), (16, 0), (16, 64), (17, 128), (31, 257), (32, 512), (33, 511),
+                                        (63, 256), (64, 129), (65, 255), (127, 1), (128, 64), (137, 63), (1024, 17),
+                                        (1025, 300), (1030, 513)])
+def test_cu_seqlens_rows_in_flight(kvt_pkg, batch, topk):
+    """The counts at the edges of the choices by rows and columns: fewer rows than wavefronts, one row or several rows
+    per wavefront at a time with groups cut off at the last row, and chunks ending at and beside a row's end."""
+    test_cu_seqlens_kernel(kvt_pkg, batch, topk, batch % 2 == 0, False)
