@@ -27,8 +27,9 @@
 // 0 <= indices[b][c] < seq_lens[b] - the columns the reference's gather writes and its attention reads when the
 // valid positions come first (the indexer pads with -1 at the end).
 //
-// What bounds it: instruction issue, most of it the exact dequantization (per tile ~460 vector instructions, 24
-// products, 72 LDS accesses, 32 loads).  Two rows per wavefront instruction (8 channels a lane), no products with
+// What bounds it: instruction issue, most of it the exact dequantization.  Counted per tile and wavefront over the paged
+// prefix chunk, resolve and merge included: 546 vector instructions (24 of them products; 692 with smoothing products),
+// 51 LDS accesses, 35 vector-memory and 30 scalar instructions, in 5,750 cycles of which 3,030 issue.  Two rows per wavefront instruction (8 channels a lane), no products with
 // smoothing factors of 1, 32-deep products (the matrix pipe takes as long for a 16-deep one) and the next tile's loads
 // in flight beside a tile's work took the paged prefix chunk (60,000 + 1,024 positions, top 2,051, 12 heads) from 237 to
 // 169 us, the dense slot decode (4 x 65,536) from 70 to 55 us and the top-k decode (8 x 2,051, 12 layers) from 234 to
