@@ -905,8 +905,8 @@ def lazy_workload(args) -> dict:
     seq_lens = torch.full((B,), CTXB, dtype=torch.int32, device="cuda")
     cu_k = torch.tensor([i * TOPK for i in range(B + 1)], dtype=torch.int32, device="cuda")
     cu_p = torch.tensor([i * CTXB for i in range(B + 1)], dtype=torch.int32, device="cuda")
-    q = [(torch.randn(B, hq, D, device="cuda", generator=g) / 4).to(torch.bfloat16) for _ in range(LAYERS)]
-    outs = [torch.empty(B, hq, D, dtype=torch.float32, device="cuda") for _ in range(LAYERS)]
+    q = [(torch.randn(B, HQ, D, device="cuda", generator=g) / 4).to(torch.bfloat16) for _ in range(LAYERS)]
+    outs = [torch.empty(B, HQ, D, dtype=torch.float32, device="cuda") for _ in range(LAYERS)]
     scr_k = torch.empty(SIZE, H, D, dtype=torch.bfloat16, device="cuda")
     scr_v = torch.empty_like(scr_k)
 

@@ -308,3 +308,27 @@ def test_stream_handle_without_the_private_query(kvt_pkg, monkeypatch):
     monkeypatch.setattr(torch, "zeros", lambda n, **k: types.SimpleNamespace(numel=lambda: n))
     kvt.prefill_workspace(torch.device("cuda", 1), 64)
     assert list(kvt._prefill_ws) == [(1, 101)]
+
+
+def test_bench_names_resolve(kvt_pkg):
+    """Every global name that bench.py's functions read exists in the module or among the builtins (its workloads run on
+    a GPU only, where a missing name would show first)."""
+    import builtins
+    import dis
+    import importlib.util
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    spec = importlib.util.spec_from_file_location("_bench_names", os.path.join(root, "bench.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+
+    def missing(code):
+        for ins in dis.get_instructions(code):
+            if ins.opname == "LOAD_GLOBAL" and not hasattr(mod, ins.argval) and not hasattr(builtins, ins.argval):
+                yield code.co_name, ins.argval
+        for const in code.co_consts:
+            if hasattr(const, "co_consts"):
+                yield from missing(const)
+
+    codes = [f.__code__ for f in vars(mod).values() if getattr(f, "__module__", None) == mod.__name__ and hasattr(f, "__code__")]
+    assert codes and [m for c in codes for m in missing(c)] == []
