@@ -98,7 +98,7 @@ KVT_DEV uint4 dequant4(const Raw& r, const float m[8]) {   // ((b & 15) - 8) * s
 // (32.5 -> 30.7).  A reader bound by the bytes of a large prefix scratch pays: non-temporal rows are not found in the
 // memory-side cache (60,000 x 16 queries 280 -> 286, sums over 71,532 rows 86.3 -> 92.9).  Gathers into a scratch of their
 // own each time gain most, since the output does not push the pools out of that cache (71,532 tokens 48.6 -> 31.1, repeated;
-// as long on a first pass).
+// a first pass 69-77 -> 68-71).
 KVT_DEV void st_out(uint16_t* p, uint4 v) {
   typedef uint32_t u4v __attribute__((ext_vector_type(4)));
   __builtin_nontemporal_store((u4v){v.x, v.y, v.z, v.w}, reinterpret_cast<u4v*>(p));
